@@ -87,6 +87,27 @@ def test_block_sparse_matches_closed_form(dev, oracle, B, Hq, Hkv, S, D, qn, kn)
                 assert (got[b, h, r0:r1] == 0).all()
 
 
+@pytest.mark.parametrize("Hq,Hkv,qn,D", [(1, 1, 1, 128), (3, 3, 15, 128), (10, 5, 16, 128), (9, 9, 17, 128), (11, 11, 33, 128)])
+def test_tile_order_reaches_every_tile(dev, oracle, Hq, Hkv, qn, D):
+    """Tile counts around the 16 tiles of one turn over the XCDs, head counts that leave the
+    last turn uneven: every row of every head is written once, by its own tile."""
+    from sparsepr_amd.kmeans_utils import dynamic_block_sparse_fwd_flashinfer
+
+    rng = np.random.default_rng(100 * Hq + qn)
+    S = 12 * qn + 5
+    q, k, v, m, qs, ks = _problem(oracle, rng, 1, Hq, Hkv, S, D, qn, 7)
+    qs = np.full_like(qs, 12)  # every q-cluster one tile, the last row count uneven
+    qs[..., -1] += 5
+    out = dynamic_block_sparse_fwd_flashinfer(
+        to_dev(q, dev, torch.bfloat16), to_dev(k, dev, torch.bfloat16), to_dev(v, dev, torch.bfloat16),
+        torch.from_numpy(m), torch.from_numpy(qs).int(), torch.from_numpy(ks).int(), is_cpu=True,
+        num_kv_heads=Hkv if Hkv != Hq else None)
+    ref, _ = _reference(oracle, q, k, v, m, qs, ks)
+    got = out.float().cpu().numpy()
+    assert np.abs(got - ref).max() <= ATOL
+    assert _cos(got, ref) >= COS
+
+
 @pytest.mark.parametrize("D,f16,Hq,Hkv", [(16, False, 2, 2), (32, False, 4, 2), (16, True, 2, 2), (32, True, 2, 2),
                                          (64, True, 4, 2), (128, True, 2, 2)])
 def test_block_sparse_head_dims_and_fp16(dev, oracle, D, f16, Hq, Hkv):
