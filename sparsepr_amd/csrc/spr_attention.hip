@@ -28,9 +28,9 @@
 // (key(t, h, e) = 16t + 8(e/4) + 4h + e%4), which makes P a plain slice of the
 // accumulator.
 //
-// Kernels: attn_pipe_kernel (D = 128 block-sparse: 256-row tiles, K/V DMA'd
+// Kernels: attn_pipe_kernel (D = 128 and 64 block-sparse: 256-row tiles, K/V DMA'd
 // into swizzled LDS tiles, next-S/softmax pipelining) and attn_fwd_kernel
-// (D = 64 block-sparse and the dense probe attention: 128-row tiles, K/V
+// (D = 16 and 32 block-sparse and the dense probe attention: 128-row tiles, K/V
 // staged through registers into a padded K tile and a transposed V tile,
 // double-buffered, the next chunk fetched while the current one computes).
 #include "spr_common.h"
@@ -746,7 +746,7 @@ __global__ __launch_bounds__(NW * 64, QB == 2 ? 1 : 2) void attn_fwd_kernel(
   }
 }
 
-// ---------------------------------------------------------------------------- block-sparse, D = 128: LDS layout
+// ---------------------------------------------------------------------------- block-sparse, D = 128 and 64: LDS layout
 // K and V chunks are copied from HBM straight into LDS (buffer_load ... lds, 16
 // bytes a lane, 1 KB per wave instruction): no staging registers and no staging
 // work in the waves' instruction streams.
@@ -765,14 +765,49 @@ __global__ __launch_bounds__(NW * 64, QB == 2 ? 1 : 2) void attn_fwd_kernel(
 // accumulator produces (key(t, h, e) = 16t + 8(e/4) + 4h + e%4).  The 4 rows x
 // 4 pieces each half-wave reads (pieces 4b .. 4b + 3) land in 16 distinct
 // slots, all 64 banks.
-constexpr int DROW = 256;         // bytes per key row (D = 128)
-constexpr int DTILE = BN * DROW;  // bytes per K or V chunk tile
+//
+// D = 64: rows of 128 bytes, two of which span the banks, so the row pair is what the
+// swizzle uses: piece j of row r at slot j ^ ((r >> 1) & 7) in K and j ^ 4((r >> 1) & 1) in V
+// (rows r and r + 1 already lie 32 banks apart).
+template <int D>
+struct PipeTile {
+  static_assert(D == 64 || D == 128, "swizzles for 128- and 256-byte rows");
+  static constexpr int ROW = 2 * D;           // bytes per key row
+  static constexpr int BYTES = BN * ROW;      // bytes per K or V chunk tile
+  static constexpr int PIECES = ROW / 16;     // 16-byte pieces per row
+  static constexpr int DMA_ROWS = 64 / PIECES;  // rows one wave's DMA instruction moves
+  __device__ static __forceinline__ int k_swz(int r) { return D == 128 ? r & 15 : (r >> 1) & 7; }
+  __device__ static __forceinline__ int v_swz(int r) { return D == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2; }
+};
 
-__device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t r, uint8_t* lds, int32_t voff) {
+typedef int32_t i32x4_s __attribute__((ext_vector_type(4)));
+
+// A raw buffer descriptor of `bytes` bytes at p, in scalar registers.
+__device__ __forceinline__ i32x4_s buffer_desc(const void* p, int32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  return i32x4_s{__builtin_amdgcn_readfirstlane(static_cast<int32_t>(a)),
+                 __builtin_amdgcn_readfirstlane(static_cast<int32_t>((a >> 32) & 0xffff)),
+                 __builtin_amdgcn_readfirstlane(bytes), 0x00020000};
+}
+
+// 16 bytes a lane from buffer offset voff to lds + 16 * lane (lds wave-uniform).  Written out
+// because the compiler tracks the builtin's write to LDS: it then waits for every DMA in
+// flight at each barrier and before most LDS reads of the tiles, which ends the prefetch.
+// Nothing tracks this one: a reader waits by s_waitcnt vmcnt and a barrier.
+__device__ __forceinline__ void lds_dma16(i32x4_s desc, const uint8_t* lds, int32_t voff) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
+  const int32_t base = __builtin_amdgcn_readfirstlane(
+      static_cast<int32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)lds)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(base), "v"(voff), "s"(desc) : "memory");
 #endif
 }
+
+// Workgroup barrier behind this wave's LDS accesses, with no wait for the DMA in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <int N>
+__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 struct alignas(8) u32x2 {
   uint32_t x, y;
@@ -788,7 +823,7 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint8_t* p) {
 #endif
 }
 
-// ---------------------------------------------------------------------------- block-sparse, D = 128, pipelined
+// ---------------------------------------------------------------------------- block-sparse, D = 128 and 64, pipelined
 // The work items, plan walk and online softmax of attn_fwd_kernel MODE 0 over
 // 256-row query tiles: eight waves of 32 rows (two per SIMD, one workgroup per
 // CU) share each K/V chunk, which halves the HBM/L2 traffic and DMA issue per
@@ -801,27 +836,34 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint8_t* p) {
 // reads the next chunk's K tile, so the chunk barrier sits before that block
 // and four LDS buffers rotate: chunk x is DMA'd right after the barrier of
 // chunk x - 3 (its buffer's previous chunk, x - 4, was last read before it)
-// and waited for before the barrier of chunk x - 1, two chunks later; key rows
-// are planned four chunks ahead.
-constexpr int TILE_RUN = 2;  // consecutive tiles of a head on one XCD
+// and waited for before the barrier of chunk x - 1, two chunks later.
+constexpr int TILE_RUN = 8;  // consecutive tiles of a head on one XCD
 // turns of TILE_RUN tiles to each of the 8 XCDs that cover a head's tiles
 __host__ __device__ inline int32_t tile_turns(int64_t tiles) {
   return static_cast<int32_t>((tiles + 8 * TILE_RUN - 1) / (8 * TILE_RUN));
 }
 
-template <bool SEGL, bool KIDX, bool F16>
-__global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
+template <int D, bool KIDX, bool F16>
+__global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int32_t s_q,
     int32_t s_kv, int32_t group, int32_t qn, int32_t kn, const int32_t* __restrict__ plan, int32_t bh_q,
     int32_t tiles_per_head, float scale_log2, const int32_t* __restrict__ q_index,
     const int32_t* __restrict__ k_index, uint16_t* __restrict__ out, float* __restrict__ lse) {
   constexpr int NW = 8;
-  constexpr int D = 128;
+  // D = 128: S of the next half is computed beside the softmax of the current one, two waves
+  // per SIMD.  D = 64: half the MFMAs meet the same softmax, which is then the bound; the plain
+  // S, softmax, P V order leaves registers for four waves per SIMD (two workgroups per CU)
+  // that cover one another (12 heads x 40,000 tokens, density 0.2: 1.26 to 1.39 ms, box to box,
+  // as the register-staged kernel took; computed ahead it is 15 % slower at two waves and
+  // 31 % at four, with spills).
+  constexpr bool AHEAD = D == 128;
+  using T = PipeTile<D>;
+  constexpr int DROW = T::ROW;
+  constexpr int DTILE = T::BYTES;
   constexpr int KSTEPS = D / 16;
   constexpr int DBLK = D / 32;
-  constexpr int NT = NW * 64;
   constexpr int TBM = NW * 32;
-  constexpr int DMA_PER_WAVE = 16 / NW;
+  constexpr int DMA_PER_WAVE = BN / T::DMA_ROWS / NW;
   __shared__ __attribute__((aligned(1024))) uint8_t k_tiles[4][DTILE];
   uint8_t* const k_tile0 = k_tiles[0];
   uint8_t* const k_tile1 = k_tiles[1];
@@ -832,23 +874,21 @@ __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
   uint8_t* const v_tile1 = v_tiles[1];
   uint8_t* const v_tile2 = v_tiles[2];
   uint8_t* const v_tile3 = v_tiles[3];
-  __shared__ int32_t key_rows[4][BN];
-  __shared__ Seg seg_lds[SEGL ? MAX_LDS_SEGS : 1];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31;
   const int half = lane >> 5;
 
   // ---- work item: workgroup b runs on XCD b % 8.  The heads follow one another and every
-  // head's 256-row tiles go to the XCDs in turn, TILE_RUN at a time (tiles of one q-cluster
-  // read the same keys and mostly share an L2), the first XCD moving on by one per head, so
-  // no XCD collects the longest tiles or the short last turn of every head.  The XCDs end
-  // together whatever the number of heads; with whole heads dealt to XCDs, 5 heads of 40,000
-  // tokens (64 x 300 clusters, density 0.2) took 1.05 ms instead of 0.93, and 24 heads of
-  // 119,056 (302 x 1,002, density 0.22) 44.4 ms instead of 42.4.  Runs of 1, 2 and 4 tiles
-  // are equal at both, 8 is 2 to 4 % slower.
+  // head's 256-row tiles go to the XCDs in turn, TILE_RUN at a time, the first XCD moving on by
+  // one per head: the XCDs end together whatever the number of heads, all of them read the
+  // same head's keys (61 MB at 118,800 tokens, which the 256 MB last-level cache holds; eight
+  // heads it does not), and the tiles of a q-cluster mostly share an L2.  Against whole heads
+  // dealt to XCDs: 5 heads of 40,000 tokens (64 x 300 clusters, density 0.2) 1.09 -> 0.99 ms,
+  // 24 heads of 119,056 (302 x 1,002, density 0.22) 45.5 -> 42.5 ms, the 24 x 118,800-token
+  // layer 36.9 ms on both.  Runs of 2 instead of 8 cost that layer 1.5 %, of 4 0.5 %.
   const int32_t per_head = tile_turns(tiles_per_head) * TILE_RUN;
   const int64_t seq = blockIdx.x / 8;
   const int64_t bhq = seq / per_head;
@@ -886,18 +926,13 @@ __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
   const int duo_part = wave >> 1;  // duo: 0 .. 3 = half + 2 (chunk parity); part 0 merges
   const bool wave_live = blk < nblk;
   const Seg* segs = pv.segs + static_cast<int64_t>(qc) * kn;
-  const int32_t nseg = pv.nseg[qc];
-  const int32_t total = pv.total[qc];
+  const int32_t nseg = __builtin_amdgcn_readfirstlane(pv.nseg[qc]);
+  const int32_t total = __builtin_amdgcn_readfirstlane(pv.total[qc]);
 
   const uint16_t* qb = q + bhq * static_cast<int64_t>(s_q) * D;
   const int32_t kv_bytes = s_kv * D * 2;
-  const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(k + bhkv * static_cast<int64_t>(s_kv) * D), 0, kv_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(v + bhkv * static_cast<int64_t>(s_kv) * D), 0, kv_bytes, 0x00020000);
-  if constexpr (SEGL) {
-    for (int i = tid; i < nseg; i += NT) seg_lds[i] = segs[i];
-  }
+  const i32x4_s k_desc = buffer_desc(k + bhkv * static_cast<int64_t>(s_kv) * D, kv_bytes);
+  const i32x4_s v_desc = buffer_desc(v + bhkv * static_cast<int64_t>(s_kv) * D, kv_bytes);
 
   int32_t my_row = row0 + blk * 32 + col;
   bool row_live = my_row < row1;
@@ -905,12 +940,12 @@ __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
     my_row = q_index[bhq * static_cast<int64_t>(s_q) + my_row];
     row_live = my_row >= 0 && my_row < s_q;
   }
+  // a dead row reads row 0 (its results are not stored): unconditional, so that the loads
+  // overlap
   u32x4 qf[KSTEPS];
+  const uint16_t* qrow = qb + static_cast<int64_t>(row_live ? my_row : 0) * D + half * 8;
 #pragma unroll
-  for (int s = 0; s < KSTEPS; ++s) {
-    qf[s] = row_live ? *reinterpret_cast<const u32x4*>(qb + static_cast<int64_t>(my_row) * D + s * 16 + half * 8)
-                     : u32x4{0, 0, 0, 0};
-  }
+  for (int s = 0; s < KSTEPS; ++s) qf[s] = *reinterpret_cast<const u32x4*>(qrow + s * 16);
   spr::f32x16 o_acc[DBLK];
 #pragma unroll
   for (int b = 0; b < DBLK; ++b) o_acc[b] = spr::f32x16{};
@@ -923,49 +958,62 @@ __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
 
   const int nch = (total + BN - 1) / BN;
 
-  int32_t cur_s = 0;
-  auto plan_chunk = [&](int c) {
-    if (wave == 0) {
-      const int32_t vpos = min(c * BN + lane, total - 1);
-      int32_t s = cur_s;
-      if constexpr (SEGL) {
-        while (s < nseg - 1 && vpos >= seg_lds[s].vend) ++s;
-      } else {
-        while (s < nseg - 1 && vpos >= segs[s].vend) ++s;
-      }
-      int32_t delta;
-      if constexpr (SEGL) delta = seg_lds[s].delta; else delta = segs[s].delta;
-      if constexpr (KIDX) {
-        key_rows[c % 4][lane] = k_index[bhkv * static_cast<int64_t>(s_kv) + delta + vpos];
-      } else {
-        key_rows[c % 4][lane] = delta + vpos;
-      }
-      cur_s = __builtin_amdgcn_readlane(s, 63);
-    }
-  };
+  // Key rows of chunk c, chunk after chunk.  The walk is scalar: lane l holds segment
+  // win_base + l of the list, the segment at the chunk's start is in scalar registers, and each
+  // segment that ends inside the chunk moves the delta of the rows past it.  No LDS or memory
+  // latency but one load per 64 segments, and every wave plans the rows it moves; each
+  // lane searching its own rows through LDS took 1 to 4 % longer on the 24 x 118,800-token
+  // layer, one wave planning for all 1.5 % longer at 302 x 1,002 clusters.
+  int32_t win_base = 0, cur_i = 0, cur_end = 0, cur_delta = 0;
+  Seg win{0, 0};
   int32_t krow[DMA_PER_WAVE];
-  auto load_rows = [&](int c) {
-    const int32_t* kr = key_rows[c % 4];
-#pragma unroll
-    for (int i = 0; i < DMA_PER_WAVE; ++i) krow[i] = kr[4 * wave + 4 * NW * i + (lane >> 4)];
+  // loaded and waited for here: a wait left to the readlanes would drain the DMA at each
+  auto load_win = [&] {
+    win = segs[min(win_base + lane, nseg - 1)];
+    asm volatile("" : "+v"(win.delta), "+v"(win.vend));
   };
-  auto dma = [&](uint8_t* kt, uint8_t* vt) {
-    const int slot = lane & 15;
+  auto load_rows = [&](int c) {
+    int32_t vpos[DMA_PER_WAVE];
 #pragma unroll
     for (int i = 0; i < DMA_PER_WAVE; ++i) {
-      const int r0 = 4 * wave + 4 * NW * i;
-      const int row = r0 + (lane >> 4);
+      vpos[i] = min(c * BN + T::DMA_ROWS * (wave + NW * i) + lane / T::PIECES, total - 1);
+      krow[i] = cur_delta;
+    }
+    // the list's last end is `total`, so the walk stays inside it
+    const int32_t chunk_end = min((c + 1) * BN, total);
+    while (cur_end < chunk_end) {
+      if (++cur_i - win_base == 64) {
+        win_base = cur_i;
+        load_win();
+      }
+      cur_delta = __builtin_amdgcn_readlane(win.delta, cur_i - win_base);
+#pragma unroll
+      for (int i = 0; i < DMA_PER_WAVE; ++i) krow[i] = vpos[i] >= cur_end ? cur_delta : krow[i];
+      cur_end = __builtin_amdgcn_readlane(win.vend, cur_i - win_base);
+    }
+#pragma unroll
+    for (int i = 0; i < DMA_PER_WAVE; ++i) {
+      krow[i] += vpos[i];
+      if constexpr (KIDX) krow[i] = k_index[bhkv * static_cast<int64_t>(s_kv) + krow[i]];
+    }
+  };
+  auto dma = [&](uint8_t* kt, uint8_t* vt) {
+    const int slot = lane % T::PIECES;
+#pragma unroll
+    for (int i = 0; i < DMA_PER_WAVE; ++i) {
+      const int r0 = T::DMA_ROWS * (wave + NW * i);
+      const int row = r0 + lane / T::PIECES;
       const int32_t off = krow[i] * DROW;
-      lds_dma16(k_rsrc, kt + r0 * DROW, off + ((slot ^ (row & 15)) << 4));
-      lds_dma16(v_rsrc, vt + r0 * DROW, off + ((slot ^ ((row & 3) << 2)) << 4));
+      lds_dma16(k_desc, kt + r0 * DROW, off + ((slot ^ T::k_swz(row)) << 4));
+      lds_dma16(v_desc, vt + r0 * DROW, off + ((slot ^ T::v_swz(row)) << 4));
     }
   };
 
-  const int k_x = half ^ (col & 15);
+  const int k_x = half ^ T::k_swz(col);
   const int tr_a = lane & 3, tr_i = (lane >> 2) & 3, tr_g = (lane >> 4) & 1;
   const int v_lane = (4 * half + tr_i) * DROW + (tr_a & 1) * 8;
   const int v_piece = 2 * tr_g + (tr_a >> 1);
-  const int v_x = 4 * tr_i;
+  const int v_x = T::v_swz(tr_i);
 
   auto s_mma = [&](spr::f32x16& acc, const uint8_t* kt, int kbk) {
     acc = spr::f32x16{};
@@ -1028,19 +1076,21 @@ __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
     for (int st = 0; st < KSTEPS; ++st) {
       if (st + 2 < KSTEPS) ka[(st + 2) % 3] = kfrag(st + 2);
       acc_next = mfma16<F16>(ka[st % 3], qf[st], acc_next);
-      const int e = 2 * st;
-      const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[e], scale_log2, neg_m));
-      const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[e + 1], scale_log2, neg_m));
-      const uint32_t pk = pack2t<F16>(p0, p1);
-      pf[e / 8][(e % 8) / 2] = pk;
-      if (e % 4 == 0) {
-        lsum0 = dot2_ones<F16>(pk, lsum0);
-      } else {
-        lsum1 = dot2_ones<F16>(pk, lsum1);
+#pragma unroll
+      for (int e = 16 / KSTEPS * st; e < 16 / KSTEPS * (st + 1); e += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[e], scale_log2, neg_m));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[e + 1], scale_log2, neg_m));
+        const uint32_t pk = pack2t<F16>(p0, p1);
+        pf[e / 8][(e % 8) / 2] = pk;
+        if (e % 4 == 0) {
+          lsum0 = dot2_ones<F16>(pk, lsum0);
+        } else {
+          lsum1 = dot2_ones<F16>(pk, lsum1);
+        }
       }
     }
     l_run += lsum0 + lsum1;
-    auto vfrag = [&](int f) {  // f = 4 tt + b
+    auto vfrag = [&](int f) {  // f = DBLK tt + b
       const uint8_t* vrow = vt + 16 * (kbk * 2 + f / DBLK) * DROW + v_lane + (((4 * (f % DBLK) + v_piece) ^ v_x) << 4);
       const u32x2 r0 = lds_read_tr16(vrow);
       const u32x2 r1 = lds_read_tr16(vrow + 8 * DROW);
@@ -1099,40 +1149,40 @@ __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
       row_max(s_a, 0, left);
       step(s_b, kt, 1, s_a, vt, 0);
     }
-    if (x + 4 < nch) plan_chunk(x + 4);
     if (x + 3 < nch) load_rows(x + 3);
     // ---- second half (S in s_b); S of the next chunk's first half goes to s_a
     if (wave_live) row_max(s_b, 1, left);
     // this wave's DMA of chunk x + 1 landed (that of chunk x + 2, issued later, may not have)
-    if (x + 2 < nch) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DMA_PER_WAVE) : "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    __syncthreads();  // ... every wave's; and no wave reads chunk x - 1 any more
+    if (x + 2 < nch) wait_vm<2 * DMA_PER_WAVE>(); else wait_vm<0>();
+    lds_barrier();  // ... every wave's; and no wave reads chunk x - 1 any more
     if (wave_live) step(s_a, kt1, 0, s_b, vt, 1);
     // chunk x + 3 into chunk x - 1's tiles, issued after this chunk's compute rather than
     // at the barrier, where every wave starts reading the next K tile (same-box timing:
-    // about 2 % faster)
+    // 1 to 2 % faster)
     if (x + 3 < nch) dma(kt3, vt3);
   };
 
-  if (nch > 0 && duo) {
-    // Step j computes chunks 2j and 2j + 1 (buffers (2j) & 3, (2j + 1) & 3) while chunks
-    // 2j + 2 and 2j + 3 land in the other two buffers, whose chunks the step before
-    // finished; key rows are planned four chunks ahead.
-    if constexpr (SEGL) __syncthreads();  // staged segment list visible to wave 0
-    for (int c = 0; c < 4 && c < nch; ++c) plan_chunk(c);
-    __syncthreads();
+  // the query rows are in registers before the first DMA: otherwise the compiler, which does
+  // not see the loops' own waits, drains the DMA before every use of them
+#pragma unroll
+  for (int st = 0; st < KSTEPS; ++st) asm volatile("" : "+v"(qf[st].x), "+v"(qf[st].y), "+v"(qf[st].z), "+v"(qf[st].w));
+  if (nch > 0) {
+    load_win();
+    cur_end = __builtin_amdgcn_readfirstlane(win.vend);
+    cur_delta = __builtin_amdgcn_readfirstlane(win.delta);
     load_rows(0);
     dma(k_tile0, v_tile0);
     if (nch > 1) {
       load_rows(1);
       dma(k_tile1, v_tile1);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  if (nch > 0 && duo) {
+    // Step j computes chunks 2j and 2j + 1 (buffers (2j) & 3, (2j + 1) & 3) while chunks
+    // 2j + 2 and 2j + 3 land in the other two buffers, whose chunks the step before finished.
     for (int x = 0; x < nch; x += 2) {
-      __syncthreads();  // chunks x, x + 1 landed for every wave; chunks x - 2, x - 1 are done
+      wait_vm<0>();   // this wave's chunks x, x + 1 landed
+      lds_barrier();  // ... every wave's; chunks x - 2, x - 1 are done
       if (x + 2 < nch) {
         load_rows(x + 2);
         dma(k_tiles[(x + 2) & 3], v_tiles[(x + 2) & 3]);
@@ -1147,54 +1197,57 @@ __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
         row_max(s_a, only, total - c * BN);
         pv_step(s_a, v_tiles[c & 3], only);
       }
-      if (x + 4 < nch) plan_chunk(x + 4);
-      if (x + 5 < nch) plan_chunk(x + 5);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's chunks x + 2, x + 3 landed
     }
   } else if (nch > 0) {
-    if constexpr (SEGL) __syncthreads();  // staged segment list visible to wave 0
-    for (int c = 0; c < 4 && c < nch; ++c) plan_chunk(c);
-    __syncthreads();
-    load_rows(0);
-    dma(k_tile0, v_tile0);
-    if (nch > 1) {
-      load_rows(1);
-      dma(k_tile1, v_tile1);
-    }
     if (nch > 2) {
       load_rows(2);
       dma(k_tile2, v_tile2);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();  // chunks 0 .. 2 landed
-    if (wave_live) s_mma(s_a, k_tile0, only);
-    if (split) {
-      // One half per chunk: S of this wave's half of chunk x is in s_a; S of the same half
-      // of chunk x + 1 (the next K tile, so after the barrier) goes to s_b.  The barriers,
-      // DMAs and planning are those of the full path.
-      for (int x = 0; x < nch; ++x) {
-        const int32_t left = total - x * BN;
-        if (x + 4 < nch) plan_chunk(x + 4);
-        if (x + 3 < nch) load_rows(x + 3);
-        if (wave_live) row_max(s_a, only, left);
-        if (x + 2 < nch) {
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DMA_PER_WAVE) : "memory");
-        } else {
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (AHEAD) {
+      wait_vm<0>();
+      lds_barrier();  // chunks 0 .. 2 landed
+      if (wave_live) s_mma(s_a, k_tile0, only);
+      if (split) {
+        // One half per chunk: S of this wave's half of chunk x is in s_a; S of the same half
+        // of chunk x + 1 (the next K tile, so after the barrier) goes to s_b.  The barriers,
+        // DMAs and planning are those of the full path.
+        for (int x = 0; x < nch; ++x) {
+          const int32_t left = total - x * BN;
+          if (x + 3 < nch) load_rows(x + 3);
+          if (wave_live) row_max(s_a, only, left);
+          if (x + 2 < nch) wait_vm<2 * DMA_PER_WAVE>(); else wait_vm<0>();
+          lds_barrier();
+          if (wave_live) {
+            step(s_b, k_tiles[(x + 1) & 3], only, s_a, v_tiles[x & 3], only);
+            s_a = s_b;
+          }
+          if (x + 3 < nch) dma(k_tiles[(x + 3) & 3], v_tiles[(x + 3) & 3]);
         }
-        __syncthreads();
-        if (wave_live) {
-          step(s_b, k_tiles[(x + 1) & 3], only, s_a, v_tiles[x & 3], only);
-          s_a = s_b;
+      } else {
+        for (int x = 0; x < nch; x += 4) {
+          chunk(x, k_tile0, v_tile0, k_tile1, k_tile3, v_tile3);
+          if (x + 1 < nch) chunk(x + 1, k_tile1, v_tile1, k_tile2, k_tile0, v_tile0);
+          if (x + 2 < nch) chunk(x + 2, k_tile2, v_tile2, k_tile3, k_tile1, v_tile1);
+          if (x + 3 < nch) chunk(x + 3, k_tile3, v_tile3, k_tile0, k_tile2, v_tile2);
         }
-        if (x + 3 < nch) dma(k_tiles[(x + 3) & 3], v_tiles[(x + 3) & 3]);
       }
     } else {
-      for (int x = 0; x < nch; x += 4) {
-        chunk(x, k_tile0, v_tile0, k_tile1, k_tile3, v_tile3);
-        if (x + 1 < nch) chunk(x + 1, k_tile1, v_tile1, k_tile2, k_tile0, v_tile0);
-        if (x + 2 < nch) chunk(x + 2, k_tile2, v_tile2, k_tile3, k_tile1, v_tile1);
-        if (x + 3 < nch) chunk(x + 3, k_tile3, v_tile3, k_tile0, k_tile2, v_tile2);
+      for (int x = 0; x < nch; ++x) {
+        // this wave's DMA of chunk x landed; those of chunks x + 1 and x + 2 may be in flight
+        if (x + 2 < nch) wait_vm<4 * DMA_PER_WAVE>(); else if (x + 1 < nch) wait_vm<2 * DMA_PER_WAVE>(); else wait_vm<0>();
+        lds_barrier();  // ... every wave's; and no wave reads chunk x - 1, whose tiles are next
+        if (x + 3 < nch) {
+          load_rows(x + 3);
+          dma(k_tiles[(x + 3) & 3], v_tiles[(x + 3) & 3]);
+        }
+        if (wave_live) {
+          const int32_t left = total - x * BN;
+          for (int h = only; h < (split ? only + 1 : 2); ++h) {
+            s_mma(s_a, k_tiles[x & 3], h);
+            row_max(s_a, h, left);
+            pv_step(s_a, v_tiles[x & 3], h);
+          }
+        }
       }
     }
   }
@@ -1537,25 +1590,24 @@ extern "C" int spr_block_sparse_attention_run_ex(const void* q, const void* k, c
   const int32_t* pl = static_cast<const int32_t*>(plan);
   uint16_t* o16 = static_cast<uint16_t*>(out);
   const int32_t s32 = static_cast<int32_t>(s), bhq32 = static_cast<int32_t>(bh_q);
-  if (d == 128) {
+  if (d == 128 || d == 64) {
     const int64_t max_tiles_pipe = spr::ceil_div(s, 2 * BM) + qn;
     const int64_t pipe_blocks = static_cast<int64_t>(tile_turns(max_tiles_pipe)) * TILE_RUN * 8 * bh_q;
     SPR_REQUIRE(pipe_blocks < (int64_t(1) << 31), "spr_block_sparse_attention_run: too many tiles");
     dim3 grid_pipe(static_cast<uint32_t>(pipe_blocks));
     const int32_t tph = static_cast<int32_t>(max_tiles_pipe);
-    auto pipe = [&](auto sl, auto kxc, auto f) {
-      attn_pipe_kernel<decltype(sl)::value, decltype(kxc)::value, decltype(f)::value><<<grid_pipe, 512, 0, stream>>>(
+    auto pipe = [&](auto dd, auto kxc, auto f) {
+      attn_pipe_kernel<decltype(dd)::value, decltype(kxc)::value, decltype(f)::value><<<grid_pipe, 512, 0, stream>>>(
           q16, k16, v16, s32, s32, group, qn, kn, pl, bhq32, tph, scale_log2, q_index, k_index, o16, lse);
     };
-    using T_ = std::true_type;
-    using F_ = std::false_type;
-    if (seg_lds) {
-      if (kx) { f16 ? pipe(T_{}, T_{}, T_{}) : pipe(T_{}, T_{}, F_{}); }
-      else    { f16 ? pipe(T_{}, F_{}, T_{}) : pipe(T_{}, F_{}, F_{}); }
-    } else {
-      if (kx) { f16 ? pipe(F_{}, T_{}, T_{}) : pipe(F_{}, T_{}, F_{}); }
-      else    { f16 ? pipe(F_{}, F_{}, T_{}) : pipe(F_{}, F_{}, F_{}); }
-    }
+    auto pipe_by_flags = [&](auto dd) {
+      using T_ = std::true_type;
+      using F_ = std::false_type;
+      if (kx) { f16 ? pipe(dd, T_{}, T_{}) : pipe(dd, T_{}, F_{}); }
+      else    { f16 ? pipe(dd, F_{}, T_{}) : pipe(dd, F_{}, F_{}); }
+    };
+    if (d == 128) pipe_by_flags(std::integral_constant<int, 128>{});
+    else pipe_by_flags(std::integral_constant<int, 64>{});
     SPR_LAUNCHED("attn_pipe_kernel");
     return SPR_OK;
   }
@@ -1576,8 +1628,7 @@ extern "C" int spr_block_sparse_attention_run_ex(const void* q, const void* k, c
       else    { f16 ? fwd(dd, F_{}, F_{}, T_{}) : fwd(dd, F_{}, F_{}, F_{}); }
     }
   };
-  if (d == 64) by_flags(std::integral_constant<int, 64>{});
-  else if (d == 32) by_flags(std::integral_constant<int, 32>{});
+  if (d == 32) by_flags(std::integral_constant<int, 32>{});
   else by_flags(std::integral_constant<int, 16>{});
   SPR_LAUNCHED("attn_fwd_kernel");
   return SPR_OK;

@@ -87,9 +87,10 @@ def test_block_sparse_matches_closed_form(dev, oracle, B, Hq, Hkv, S, D, qn, kn)
                 assert (got[b, h, r0:r1] == 0).all()
 
 
-@pytest.mark.parametrize("Hq,Hkv,qn,D", [(1, 1, 1, 128), (3, 3, 15, 128), (10, 5, 16, 128), (9, 9, 17, 128), (11, 11, 33, 128)])
+@pytest.mark.parametrize("Hq,Hkv,qn,D", [(1, 1, 1, 128), (3, 3, 7, 128), (10, 5, 8, 128), (9, 9, 17, 64),
+                                          (11, 11, 33, 128), (2, 2, 65, 128)])
 def test_tile_order_reaches_every_tile(dev, oracle, Hq, Hkv, qn, D):
-    """Tile counts around the 16 tiles of one turn over the XCDs, head counts that leave the
+    """Tile counts around the 8 tiles of a run and the 64 of one turn over the XCDs, head counts that leave the
     last turn uneven: every row of every head is written once, by its own tile."""
     from sparsepr_amd.kmeans_utils import dynamic_block_sparse_fwd_flashinfer
 
@@ -106,6 +107,48 @@ def test_tile_order_reaches_every_tile(dev, oracle, Hq, Hkv, qn, D):
     got = out.float().cpu().numpy()
     assert np.abs(got - ref).max() <= ATOL
     assert _cos(got, ref) >= COS
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("rows", [31, 64, 100, 161, 256, 300])  # one to eight 32-row blocks, two tiles
+@pytest.mark.parametrize("keys", [1, 64, 65, 128, 193, 320])
+def test_block_sparse_chunk_and_tile_edges(dev, oracle, D, rows, keys):
+    """Key counts at the 64-key chunk edges and below the four chunks in flight, for every way a
+    tile's waves share its rows."""
+    from sparsepr_amd.kernels.attention import block_sparse_attention
+
+    rng = np.random.default_rng(D + rows + keys)
+    S = 330
+    q, k, v = (oracle.to_bf16(rng.standard_normal((1, 1, S, D)).astype(np.float32)) for _ in range(3))
+    qs = np.array([[[rows, S - rows]]])
+    ks = np.array([[[3, keys, S - keys - 3]]])
+    m = np.array([[[[False, True, False], [True, False, True]]]])
+    t = [to_dev(a[0], dev, torch.bfloat16) for a in (q, k, v)]
+    got = block_sparse_attention(*t, torch.from_numpy(m[0]).to(dev), torch.from_numpy(qs[0]).to(dev),
+                                 torch.from_numpy(ks[0]).to(dev))
+    ref, _ = _reference(oracle, q, k, v, m, qs, ks)
+    assert np.abs(got.float().cpu().numpy() - ref[0]).max() <= ATOL
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("kn,size", [(64, 3), (65, 3), (129, 1), (700, 1), (3, 70)])
+def test_block_sparse_segment_walk(dev, oracle, D, kn, size):
+    """Segment lists of one window of 64 and more, of one-key and of chunk-long segments (a chunk
+    holds up to 64 ends), with a row whose last segment ends inside a chunk."""
+    from sparsepr_amd.kernels.attention import block_sparse_attention
+
+    rng = np.random.default_rng(kn + size)
+    S = kn * size
+    q, k, v = (oracle.to_bf16(rng.standard_normal((1, 1, S, D)).astype(np.float32)) for _ in range(3))
+    qs = np.array([[[S // 3, S - S // 3]]])
+    ks = np.full((1, 1, kn), size)
+    m = np.ones((1, 1, 2, kn), bool)
+    m[0, 0, 1, 1::3] = False
+    t = [to_dev(a[0], dev, torch.bfloat16) for a in (q, k, v)]
+    got = block_sparse_attention(*t, torch.from_numpy(m[0]).to(dev), torch.from_numpy(qs[0]).to(dev),
+                                 torch.from_numpy(ks[0]).to(dev))
+    ref, _ = _reference(oracle, q, k, v, m, qs, ks)
+    assert np.abs(got.float().cpu().numpy() - ref[0]).max() <= ATOL
 
 
 @pytest.mark.parametrize("D,f16,Hq,Hkv", [(16, False, 2, 2), (32, False, 4, 2), (16, True, 2, 2), (32, True, 2, 2),
