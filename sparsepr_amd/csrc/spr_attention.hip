@@ -780,35 +780,6 @@ struct PipeTile {
   __device__ static __forceinline__ int v_swz(int r) { return D == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2; }
 };
 
-typedef int32_t i32x4_s __attribute__((ext_vector_type(4)));
-
-// A raw buffer descriptor of `bytes` bytes at p, in scalar registers.
-__device__ __forceinline__ i32x4_s buffer_desc(const void* p, int32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(p);
-  return i32x4_s{__builtin_amdgcn_readfirstlane(static_cast<int32_t>(a)),
-                 __builtin_amdgcn_readfirstlane(static_cast<int32_t>((a >> 32) & 0xffff)),
-                 __builtin_amdgcn_readfirstlane(bytes), 0x00020000};
-}
-
-// 16 bytes a lane from buffer offset voff to lds + 16 * lane (lds wave-uniform).  Written out
-// because the compiler tracks the builtin's write to LDS: it then waits for every DMA in
-// flight at each barrier and before most LDS reads of the tiles, which ends the prefetch.
-// Nothing tracks this one: a reader waits by s_waitcnt vmcnt and a barrier.
-__device__ __forceinline__ void lds_dma16(i32x4_s desc, const uint8_t* lds, int32_t voff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const int32_t base = __builtin_amdgcn_readfirstlane(
-      static_cast<int32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)lds)));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(base), "v"(voff), "s"(desc) : "memory");
-#endif
-}
-
-// Workgroup barrier behind this wave's LDS accesses, with no wait for the DMA in flight.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-template <int N>
-__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 struct alignas(8) u32x2 {
   uint32_t x, y;
 };
@@ -931,8 +902,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
 
   const uint16_t* qb = q + bhq * static_cast<int64_t>(s_q) * D;
   const int32_t kv_bytes = s_kv * D * 2;
-  const i32x4_s k_desc = buffer_desc(k + bhkv * static_cast<int64_t>(s_kv) * D, kv_bytes);
-  const i32x4_s v_desc = buffer_desc(v + bhkv * static_cast<int64_t>(s_kv) * D, kv_bytes);
+  const spr::i32x4_s k_desc = spr::buffer_desc(k + bhkv * static_cast<int64_t>(s_kv) * D, kv_bytes);
+  const spr::i32x4_s v_desc = spr::buffer_desc(v + bhkv * static_cast<int64_t>(s_kv) * D, kv_bytes);
 
   int32_t my_row = row0 + blk * 32 + col;
   bool row_live = my_row < row1;
@@ -1004,8 +975,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
       const int r0 = T::DMA_ROWS * (wave + NW * i);
       const int row = r0 + lane / T::PIECES;
       const int32_t off = krow[i] * DROW;
-      lds_dma16(k_desc, kt + r0 * DROW, off + ((slot ^ T::k_swz(row)) << 4));
-      lds_dma16(v_desc, vt + r0 * DROW, off + ((slot ^ T::v_swz(row)) << 4));
+      spr::lds_dma16(k_desc, kt + r0 * DROW, off + ((slot ^ T::k_swz(row)) << 4));
+      spr::lds_dma16(v_desc, vt + r0 * DROW, off + ((slot ^ T::v_swz(row)) << 4));
     }
   };
 
@@ -1153,8 +1124,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
     // ---- second half (S in s_b); S of the next chunk's first half goes to s_a
     if (wave_live) row_max(s_b, 1, left);
     // this wave's DMA of chunk x + 1 landed (that of chunk x + 2, issued later, may not have)
-    if (x + 2 < nch) wait_vm<2 * DMA_PER_WAVE>(); else wait_vm<0>();
-    lds_barrier();  // ... every wave's; and no wave reads chunk x - 1 any more
+    if (x + 2 < nch) spr::wait_vm<2 * DMA_PER_WAVE>(); else spr::wait_vm<0>();
+    spr::lds_barrier();  // ... every wave's; and no wave reads chunk x - 1 any more
     if (wave_live) step(s_a, kt1, 0, s_b, vt, 1);
     // chunk x + 3 into chunk x - 1's tiles, issued after this chunk's compute rather than
     // at the barrier, where every wave starts reading the next K tile (same-box timing:
@@ -1181,8 +1152,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
     // Step j computes chunks 2j and 2j + 1 (buffers (2j) & 3, (2j + 1) & 3) while chunks
     // 2j + 2 and 2j + 3 land in the other two buffers, whose chunks the step before finished.
     for (int x = 0; x < nch; x += 2) {
-      wait_vm<0>();   // this wave's chunks x, x + 1 landed
-      lds_barrier();  // ... every wave's; chunks x - 2, x - 1 are done
+      spr::wait_vm<0>();   // this wave's chunks x, x + 1 landed
+      spr::lds_barrier();  // ... every wave's; chunks x - 2, x - 1 are done
       if (x + 2 < nch) {
         load_rows(x + 2);
         dma(k_tiles[(x + 2) & 3], v_tiles[(x + 2) & 3]);
@@ -1204,8 +1175,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
       dma(k_tile2, v_tile2);
     }
     if constexpr (AHEAD) {
-      wait_vm<0>();
-      lds_barrier();  // chunks 0 .. 2 landed
+      spr::wait_vm<0>();
+      spr::lds_barrier();  // chunks 0 .. 2 landed
       if (wave_live) s_mma(s_a, k_tile0, only);
       if (split) {
         // One half per chunk: S of this wave's half of chunk x is in s_a; S of the same half
@@ -1215,8 +1186,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
           const int32_t left = total - x * BN;
           if (x + 3 < nch) load_rows(x + 3);
           if (wave_live) row_max(s_a, only, left);
-          if (x + 2 < nch) wait_vm<2 * DMA_PER_WAVE>(); else wait_vm<0>();
-          lds_barrier();
+          if (x + 2 < nch) spr::wait_vm<2 * DMA_PER_WAVE>(); else spr::wait_vm<0>();
+          spr::lds_barrier();
           if (wave_live) {
             step(s_b, k_tiles[(x + 1) & 3], only, s_a, v_tiles[x & 3], only);
             s_a = s_b;
@@ -1234,8 +1205,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
     } else {
       for (int x = 0; x < nch; ++x) {
         // this wave's DMA of chunk x landed; those of chunks x + 1 and x + 2 may be in flight
-        if (x + 2 < nch) wait_vm<4 * DMA_PER_WAVE>(); else if (x + 1 < nch) wait_vm<2 * DMA_PER_WAVE>(); else wait_vm<0>();
-        lds_barrier();  // ... every wave's; and no wave reads chunk x - 1, whose tiles are next
+        if (x + 2 < nch) spr::wait_vm<4 * DMA_PER_WAVE>(); else if (x + 1 < nch) spr::wait_vm<2 * DMA_PER_WAVE>(); else spr::wait_vm<0>();
+        spr::lds_barrier();  // ... every wave's; and no wave reads chunk x - 1, whose tiles are next
         if (x + 3 < nch) {
           load_rows(x + 3);
           dma(k_tiles[(x + 3) & 3], v_tiles[(x + 3) & 3]);

@@ -108,6 +108,36 @@ __device__ __forceinline__ float canonical_expf(float x) {
   return (p * sa) * sb;  // exact power-of-two scaling
 }
 
+// ---------------------------------------------------------------- LDS DMA
+typedef int32_t i32x4_s __attribute__((ext_vector_type(4)));
+
+// A raw buffer descriptor of `bytes` bytes at p, in scalar registers.
+__device__ __forceinline__ i32x4_s buffer_desc(const void* p, int32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  return i32x4_s{__builtin_amdgcn_readfirstlane(static_cast<int32_t>(a)),
+                 __builtin_amdgcn_readfirstlane(static_cast<int32_t>((a >> 32) & 0xffff)),
+                 __builtin_amdgcn_readfirstlane(bytes), 0x00020000};
+}
+
+// 16 bytes a lane from buffer offset voff to lds + 16 * lane (lds wave-uniform).  Written out
+// because the compiler tracks the builtin's write to LDS: it then waits for every DMA in
+// flight at each barrier and before most LDS reads of the tiles, which ends the prefetch.
+// Nothing tracks this one: a reader waits by s_waitcnt vmcnt and a barrier.
+__device__ __forceinline__ void lds_dma16(i32x4_s desc, const uint8_t* lds, int32_t voff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int32_t base = __builtin_amdgcn_readfirstlane(
+      static_cast<int32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)lds)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(base), "v"(voff), "s"(desc) : "memory");
+#endif
+}
+
+// Workgroup barrier behind this wave's LDS accesses, with no wait for the DMA in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <int N>
+__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
 // ---------------------------------------------------------------- misc
 __host__ __device__ __forceinline__ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

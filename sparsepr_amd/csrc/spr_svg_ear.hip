@@ -15,27 +15,35 @@
 //       E = sum_t max(w_c^2 |vc|^2 + w_t^2 |v_t|^2 - 2 w_t w_c (v_t . vc), 0)
 //       score = log(max(E / n_c, 1e-30)) + 2 m;  -inf for an empty cluster
 //   attention mass: score = log(max(sum_t e^(l_t - m), 1e-30)) + m, m = max_t l_t
-// The running max is kept per 32-token chunk with the reference's rescaling
-// (E *= alpha^2, w_c *= alpha; the mass sum *= alpha).
+// The weights are taken against a reference that starts at l_c (the mass: at the first
+// chunk's maximum) and moves only when a logit passes it by SE_SLACK, with the sums rescaled;
+// the scores do not depend on it but for rounding.
 //
-// Layout.  A first kernel writes the centroid logits l_c [query head, centroid,
-// cluster] (fp32 dot products over d, sequential, 128 rows x 32 clusters per workgroup)
-// into the score buffer; the score kernel overwrites each entry with its score.
-// The score kernel runs one workgroup of four waves per (query head, 8
-// consecutive key clusters); wave w scores query rows 32 w .. 32 w + 31 of each
-// group of 128 (a loop covers more centroids).  The clusters' tokens are one
-// contiguous run, walked in 32-token chunks (a chunk never spans two clusters).
-// Per chunk: every thread holds 32 bytes of K and of V (token tid / 8, dims
-// 16 (tid % 8) .. + 15), prefetched during the previous chunk; it stores the K
-// bytes into a swizzled LDS tile (16-byte piece p of token row t at slot
-// p ^ (t % 16): the MFMA fragment reads hit 16 distinct slots per 16 lanes) and
-// reduces |v_t|^2 and v_t . vc over the token's 8 threads (DPP) into LDS.  After one
-// barrier S^T = K Q~^T comes from 16 bf16 MFMAs per wave: q~ is split into bf16
-// hi + lo with hi + lo == q~ exactly (q~ has 11 significant bits, hi the top 8,
-// lo the next 3), so every product is the reference's TF32 product exactly and
-// only the fp32 summation order differs.  Two LDS buffers alternate by chunk.
-// The token runs come from a block prefix sum of the sizes and are clamped to
-// the stored tokens, so no size vector can make the kernel read outside K or V.
+// Layout.  A first kernel writes the centroid logits l_c [query head, centroid, cluster]
+// (fp32 dot products over d, sequential, 128 rows x 32 clusters per workgroup) into the score
+// buffer; the score kernel overwrites each entry with its score.  The score kernel runs one
+// workgroup per CU for (query head, 8 consecutive key clusters, up to 320 query rows): a wave
+// per 32-row query block (two for up to five blocks, each folding every other chunk), two
+// waves for the statistics of V, at most twelve, three per SIMD.  K and V are walked once for
+// all rows.  The clusters' tokens are one contiguous run, walked in 32-token chunks (a chunk
+// never spans two clusters), whose K and V rows are DMA'd into swizzled LDS tiles (16-byte
+// piece p of token row t at slot p ^ (t % 16): the MFMA fragment reads hit 16 distinct slots
+// per 16 lanes) two steps of two chunks ahead.  A query wave forms S^T = K Q~^T by 16 bf16
+// MFMAs per chunk: q~ is split into bf16 hi + lo with hi + lo == q~ exactly (q~ has 11
+// significant bits, hi the top 8, lo the next 3), so every product is the reference's TF32
+// product exactly and only the fp32 summation order differs.  |v_t|^2 and v_t . vc are products
+// of the V tile with itself and with the three bf16 pieces of vc, a chunk ahead of their use.
+//
+// What bounds it: the folding, 5 VALU operations, an exponential (16 cycles) and half a max
+// per (centroid, token) pair beside the MFMAs, which a wave does not overlap with its own
+// (computing S a chunk ahead needs more registers than three waves per SIMD have).  24 heads x
+// 118,800 tokens, 300 x 1000: 1.27 -> 0.94 ms; 180 x 512 at 70,000 tokens (both kernels) 0.64
+// -> 0.48 ms, 128 x 512 at 118,800 0.55 -> 0.53 ms, 6 heads x 9,000 tokens, 23 x 64: 105 -> 64
+// us, against four waves per 128 rows that walked K and V again for every 128 rows and took
+// the statistics of V on all their lanes.  One wave for the statistics instead of two holds
+// the others up (128 x 512: 0.64 ms); one chunk per barrier costs 5 %.
+// The token runs come from a block prefix sum of the sizes and are clamped to the stored
+// tokens, so no size vector can make the kernel read outside K or V.
 #include <type_traits>
 
 #include "spr_common.h"
@@ -43,11 +51,11 @@
 namespace {
 
 using spr::f32x16;
+using spr::f32x4;
 using spr::u32x4;
 
 constexpr int SE_D = 128;
 constexpr int SE_THREADS = 256;
-constexpr int SE_WAVES = SE_THREADS / 64;
 constexpr int SE_CHUNK = 32;  // tokens per chunk: one 32-row MFMA block
 constexpr int SE_KSTEPS = SE_D / 16;
 constexpr float SE_LOG2E = 1.4426950408889634f;
@@ -63,18 +71,6 @@ __device__ __forceinline__ float wave_sum(float v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
-
-__device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t r, uint8_t* lds, int32_t voff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
-#endif
-}
-
-// Workgroup barrier after this wave's LDS accesses completed, with no wait on the
-// vector memory counter: LDS DMA of later chunks stays in flight across it (its
-// landing is waited for explicitly).  The memory clobber keeps the compiler from
-// moving LDS accesses across it.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
@@ -101,21 +97,21 @@ __device__ __forceinline__ float sum_xor32(float x) {
 }
 
 constexpr int SE_ROW = SE_D * 2;  // bytes per bf16 token row
-// key clusters per workgroup (4 was faster on synthetic cluster sizes but 2 % slower on the
-// routed clusters of the C4 bench, and within noise in the N8 step; 2 and 16 were slower)
-constexpr int SE_CPW = 8;
 constexpr int CL_CLUSTERS = 32;   // clusters per centroid-logit workgroup
+constexpr int CL_PITCH = SE_D + 4;  // floats per centroid row in LDS
 constexpr int CL_ROWS = 2 * (SE_THREADS / 4);  // query rows per centroid-logit workgroup
 
 // l_c = (q . kc) / sqrt(D) (+ 0.5 min(sum_d q_d^2 var_d / D, cap)) for CL_ROWS query rows x
 // CL_CLUSTERS clusters per workgroup: thread -> query rows tid / 4 and tid / 4 + CL_ROWS / 2,
-// clusters 8 (tid % 4) .. + 7 (each centroid read from LDS serves two rows); fp32 fma chains
-// over d in order.  Written to out [qh, qn, kn].
+// clusters tid % 4 + 4 j, j < 8 (each centroid read from LDS serves two rows, and the four
+// neighbours' rows of CL_PITCH floats lie in distinct banks: 90 -> 68 us for 24 heads of
+// 300 x 1000 against clusters 8 (tid % 4) + j of unpadded rows, four to a bank); fp32 fma
+// chains over d in order.  Written to out [qh, qn, kn].
 __global__ __launch_bounds__(SE_THREADS) void svg_ear_centroid_logit_kernel(
     const float* __restrict__ qc, const float* __restrict__ kcent, const float* __restrict__ var_k, float cap,
     int32_t qn, int32_t kn, int32_t group, float* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) float kc_l[CL_CLUSTERS][SE_D];
-  __shared__ __attribute__((aligned(16))) float var_l[CL_CLUSTERS][SE_D];
+  __shared__ __attribute__((aligned(16))) float kc_l[CL_CLUSTERS][CL_PITCH];
+  __shared__ __attribute__((aligned(16))) float var_l[CL_CLUSTERS][CL_PITCH];
   const int64_t qh = blockIdx.z;
   const int64_t kh = qh / group;
   const int cb = blockIdx.x * CL_CLUSTERS;
@@ -134,7 +130,7 @@ __global__ __launch_bounds__(SE_THREADS) void svg_ear_centroid_logit_kernel(
   __syncthreads();
   const int r0 = blockIdx.y * CL_ROWS + tid / 4;
   const int r1 = r0 + CL_ROWS / 2;
-  const int c0 = 8 * (tid % 4);
+  const int c0 = tid % 4;
   if (r0 >= qn) return;
   const float* qrow0 = qc + (qh * qn + r0) * SE_D;
   const float* qrow1 = qc + (qh * qn + min(r1, qn - 1)) * SE_D;  // a row past qn computes, stores nothing
@@ -146,7 +142,7 @@ __global__ __launch_bounds__(SE_THREADS) void svg_ear_centroid_logit_kernel(
     const float4 qb = *reinterpret_cast<const float4*>(qrow1 + d0);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float4 kv = *reinterpret_cast<const float4*>(&kc_l[c0 + j][d0]);
+      const float4 kv = *reinterpret_cast<const float4*>(&kc_l[c0 + 4 * j][d0]);
       dot0[j] = __builtin_fmaf(qa.x, kv.x, dot0[j]);
       dot0[j] = __builtin_fmaf(qa.y, kv.y, dot0[j]);
       dot0[j] = __builtin_fmaf(qa.z, kv.z, dot0[j]);
@@ -156,7 +152,7 @@ __global__ __launch_bounds__(SE_THREADS) void svg_ear_centroid_logit_kernel(
       dot1[j] = __builtin_fmaf(qb.z, kv.z, dot1[j]);
       dot1[j] = __builtin_fmaf(qb.w, kv.w, dot1[j]);
       if (var_k != nullptr) {
-        const float4 vv = *reinterpret_cast<const float4*>(&var_l[c0 + j][d0]);
+        const float4 vv = *reinterpret_cast<const float4*>(&var_l[c0 + 4 * j][d0]);
         s20[j] = __builtin_fmaf(qa.x * qa.x, vv.x, s20[j]);
         s20[j] = __builtin_fmaf(qa.y * qa.y, vv.y, s20[j]);
         s20[j] = __builtin_fmaf(qa.z * qa.z, vv.z, s20[j]);
@@ -172,10 +168,10 @@ __global__ __launch_bounds__(SE_THREADS) void svg_ear_centroid_logit_kernel(
     float* orow = out + (qh * qn + r) * kn + cb + c0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      if (c0 + j < ncl) {
+      if (c0 + 4 * j < ncl) {
         float l = dot[j] * scale;
         if (var_k != nullptr) l += 0.5f * fminf(s2[j] / static_cast<float>(SE_D), cap);
-        orow[j] = l;
+        orow[4 * j] = l;
       }
     }
   };
@@ -183,166 +179,234 @@ __global__ __launch_bounds__(SE_THREADS) void svg_ear_centroid_logit_kernel(
   if (r1 < qn) store(r1, dot1, s21);
 }
 
+// Key clusters per workgroup and the most query waves of one.
+constexpr int SE_CPW = 8;
+constexpr int SE_QWAVES = 10;
+constexpr int SE_SWAVES = 2;  // waves that take the V statistics, every other chunk each
+constexpr int SE_TILES = 8;   // chunks of K in LDS
+constexpr int SE_VTILES = 6;  // chunks of V, whose statistics are taken a step ahead
+constexpr int SE_TILE = SE_CHUNK * SE_ROW;  // bytes of a K or V tile
+// a running reference is moved once a chunk's largest logit passes it by this much: the weights
+// stay below e^30, their squares times a cluster's values inside fp32
+constexpr float SE_SLACK = 30.0f;
+
 template <int MODE>  // 0: value error (scores holds l_c on entry), 1: attention mass
-__global__ __launch_bounds__(SE_THREADS) void svg_ear_score_kernel(
+__global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score_kernel(
     const float* __restrict__ qc, const uint16_t* __restrict__ ks, const uint16_t* __restrict__ vs,
     const float* __restrict__ vcent, const int32_t* __restrict__ k_sizes, int32_t qn, int32_t kn, int64_t t_stored,
-    int32_t group, float* __restrict__ scores) {
-  // four K and four V tiles as separate arrays: the chunk loop is unrolled by four so that
-  // every LDS read names a tile the compiler can tell apart from the ones being DMA'd
-  // (otherwise it waits for all DMA in flight before each read)
-  __shared__ __attribute__((aligned(1024))) uint8_t k_l0[SE_CHUNK * SE_ROW];
-  __shared__ __attribute__((aligned(1024))) uint8_t k_l1[SE_CHUNK * SE_ROW];
-  __shared__ __attribute__((aligned(1024))) uint8_t k_l2[SE_CHUNK * SE_ROW];
-  __shared__ __attribute__((aligned(1024))) uint8_t k_l3[SE_CHUNK * SE_ROW];
-  __shared__ __attribute__((aligned(1024))) uint8_t v_l0[SE_CHUNK * SE_ROW];
-  __shared__ __attribute__((aligned(1024))) uint8_t v_l1[SE_CHUNK * SE_ROW];
-  __shared__ __attribute__((aligned(1024))) uint8_t v_l2[SE_CHUNK * SE_ROW];
-  __shared__ __attribute__((aligned(1024))) uint8_t v_l3[SE_CHUNK * SE_ROW];
-  __shared__ __attribute__((aligned(16))) float vn2_l[2][SE_CHUNK];
-  __shared__ __attribute__((aligned(16))) float cdv_l[2][SE_CHUNK];
-  __shared__ float vc_l[SE_CPW][SE_D];
+    int32_t group, int32_t qgroups, int32_t qwaves, int32_t sets, float* __restrict__ scores) {
+  __shared__ __attribute__((aligned(1024))) uint8_t k_tiles[SE_TILES * SE_TILE];
+  __shared__ __attribute__((aligned(1024))) uint8_t v_tiles[MODE == 0 ? SE_VTILES * SE_TILE : 16];
+  // the value centroids as three bf16 pieces whose sum they are, and a row of zeros
+  __shared__ __attribute__((aligned(16))) uint16_t vc_l[MODE == 0 ? 3 * SE_CPW + 1 : 1][SE_D];
+  __shared__ __attribute__((aligned(16))) float vn_l[4][SE_CHUNK];  // |v_t|^2
+  __shared__ __attribute__((aligned(16))) float cd_l[4][SE_CHUNK];  // -2 v_t . vc
   __shared__ float vc2_l[SE_CPW];
-  __shared__ float cl_l[SE_CPW][32 * SE_WAVES];
-  __shared__ int32_t start_l[SE_CPW];  // first stored token of each cluster's run (clamped)
-  __shared__ int32_t len_l[SE_CPW];    // tokens in each run (clamped)
-  __shared__ int32_t nxt_l[SE_CPW];    // next cluster with tokens (ncl if none)
-  __shared__ int64_t red_l[SE_WAVES];
+  // per cluster and row of a q wave: the sum, the reference it is taken against, the largest logit
+  __shared__ float es_l[SE_CPW][32 * SE_QWAVES];
+  __shared__ float rf_l[SE_CPW][32 * SE_QWAVES];
+  __shared__ float tp_l[SE_CPW][32 * SE_QWAVES];
+  __shared__ int32_t len_l[SE_CPW];  // tokens in each run (clamped)
+  __shared__ int64_t red_l[SE_QWAVES + SE_SWAVES];
 
-  const int c_begin = blockIdx.x * SE_CPW;
+  // Workgroup b runs on XCD b % 8: the query groups of the same clusters follow one another
+  // there and find K and V in its L2.
+  const int turn = blockIdx.x / 8;
+  const int c_begin = (turn / qgroups * 8 + static_cast<int>(blockIdx.x % 8)) * SE_CPW;
+  if (c_begin >= kn) return;
+  const int q0 = turn % qgroups * (32 * qwaves);
   const int ncl = min(SE_CPW, kn - c_begin);
   const int64_t qh = blockIdx.y;
   const int64_t kh = qh / group;
   const int tid = threadIdx.x;
+  const int nthr = blockDim.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31;
   const int half = lane >> 5;
   const float scale = 1.0f / 11.313708498984761f;  // 1 / sqrt(128), as the fp32 quotient
+  // wave w < qwaves * sets folds query block w % qwaves; with two sets each folds every other
+  // chunk and the sums meet at the end
+  const int set = wave / qwaves;
+  const int q = q0 + 32 * (wave % qwaves) + col;
+  const bool q_wave = set < sets && q0 + 32 * (wave % qwaves) < qn;
+  const int stat = MODE == 0 ? wave - qwaves * sets : -1;  // 0 or 1: takes the statistics of that chunk of a step
+  const int rows = 32 * qwaves;
 
+  // the query rows on their way while the rest is set up (rows past the end read the last one,
+  // waves without a block store nothing of theirs)
+  const float* qrow = qc + (qh * qn + min(q, qn - 1)) * SE_D + 8 * half;
+  float4 qraw[2 * SE_KSTEPS];
+#pragma unroll
+  for (int s = 0; s < SE_KSTEPS; ++s) {
+    qraw[2 * s] = *reinterpret_cast<const float4*>(qrow + 16 * s);
+    qraw[2 * s + 1] = *reinterpret_cast<const float4*>(qrow + 16 * s + 4);
+  }
+  // every sum starts empty, against l_c (written by svg_ear_centroid_logit_kernel)
+  for (int i = tid; i < SE_CPW * rows; i += nthr) {
+    const int j = i % SE_CPW, r = i / SE_CPW;
+    float l = -__builtin_huge_valf();
+    if (MODE == 0 && j < ncl && q0 + r < qn) l = scores[(qh * qn + q0 + r) * kn + c_begin + j];
+    for (int t = 0; t < sets; ++t) {
+      es_l[j][t * rows + r] = 0.0f;
+      rf_l[j][t * rows + r] = l;
+      tp_l[j][t * rows + r] = l;
+    }
+  }
   // ---- token runs of clusters c_begin .. c_begin + ncl - 1 (negative sizes count as 0)
   const int32_t* sz = k_sizes + kh * kn;
+  const int32_t own = lane < ncl ? max(sz[c_begin + lane], 0) : 0;
   int64_t part = 0;
-  for (int j = tid; j < c_begin; j += SE_THREADS) part += max(sz[j], 0);
+  for (int j = tid; j < c_begin; j += nthr) part += max(sz[j], 0);
   for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
   if (lane == 0) red_l[wave] = part;
   if (MODE == 0) {
-    for (int i = tid; i < SE_CPW * SE_D; i += SE_THREADS) {
-      const int j = i / SE_D;
-      vc_l[j][i % SE_D] = j < ncl ? vcent[(kh * kn + c_begin + j) * SE_D + i % SE_D] : 0.0f;
+    for (int i = tid; i < SE_CPW * SE_D; i += nthr) {
+      const int j = i / SE_D, d = i % SE_D;
+      const float v = j < ncl ? vcent[(kh * kn + c_begin + j) * SE_D + d] : 0.0f;
+      const uint32_t hi = __float_as_uint(v) & 0xffff0000u;
+      const float r1 = v - __uint_as_float(hi);
+      const uint32_t mid = __float_as_uint(r1) & 0xffff0000u;
+      vc_l[3 * j][d] = static_cast<uint16_t>(hi >> 16);
+      vc_l[3 * j + 1][d] = static_cast<uint16_t>(mid >> 16);
+      vc_l[3 * j + 2][d] = spr::f32_to_bf16(r1 - __uint_as_float(mid));
+    }
+    for (int i = tid; i < SE_D; i += nthr) vc_l[3 * SE_CPW][i] = 0;
+    for (int j = wave; j < ncl; j += nthr / 64) {
+      const float* vr = vcent + (kh * kn + c_begin + j) * SE_D;
+      const float x = vr[2 * lane], y = vr[2 * lane + 1];
+      const float s2 = wave_sum(__builtin_fmaf(x, x, y * y));
+      if (lane == 0) vc2_l[j] = s2;
     }
   }
   __syncthreads();
-  if (tid == 0) {
-    int64_t cum = 0;
-    for (int w = 0; w < SE_WAVES; ++w) cum += red_l[w];
-    for (int j = 0; j < SE_CPW; ++j) {
-      const int64_t a = min(cum, t_stored);
-      if (j < ncl) cum += max(sz[c_begin + j], 0);
-      start_l[j] = static_cast<int32_t>(a);
-      len_l[j] = static_cast<int32_t>(min(cum, t_stored) - a);
-    }
-    int next = ncl;
-    for (int j = SE_CPW - 1; j >= 0; --j) {
-      nxt_l[j] = next;
-      if (j < ncl && len_l[j] > 0) next = j;
-    }
+  // lane j holds cluster j's run (first stored token and length, clamped); the walks are scalar
+  int64_t before = 0;
+  for (int w = 0; w < nthr / 64; ++w) before += red_l[w];
+  int64_t upto = own;
+  for (int o = 1; o < SE_CPW; o <<= 1) {
+    const int64_t up = __shfl_up(upto, o, 64);
+    if (lane >= o) upto += up;
   }
-  if (MODE == 0) {
-    for (int j = wave; j < SE_CPW; j += SE_WAVES) {
-      const float a = vc_l[j][2 * lane], b = vc_l[j][2 * lane + 1];
-      const float s = wave_sum(__builtin_fmaf(a, a, b * b));
-      if (lane == 0) vc2_l[j] = s;
-    }
-  }
-  __syncthreads();
-  auto cl_len = [&](int j) { return len_l[j]; };
-  // empty clusters score -inf
-  for (int j = 0; j < ncl; ++j) {
-    if (cl_len(j) <= 0) {
-      for (int q = tid; q < qn; q += SE_THREADS) scores[(qh * qn + q) * kn + c_begin + j] = -__builtin_huge_valf();
-    }
-  }
-  const int j_first = cl_len(0) > 0 ? 0 : nxt_l[0];
-  if (j_first >= ncl) return;
-
-  // ---- K/V chunks land in LDS by DMA: 32 token rows of 256 bytes per tile; wave w moves rows
-  // 4 w .. 4 w + 3 and 16 + 4 w .. + 3 (1 KB per instruction).  In the K tile the lane that
-  // fills slot p of row t fetches piece p ^ (t % 16) (the swizzle of the MFMA reads); V is
-  // stored as is.  Rows past the cluster's run hold the next cluster's tokens (masked in the
-  // scores); rows past the stored tokens read as zero (buffer bounds).
-  const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(ks + kh * t_stored * SE_D), 0, static_cast<int32_t>(t_stored * SE_ROW), 0x00020000);
-  const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(MODE == 0 ? vs + kh * t_stored * SE_D : ks), 0, static_cast<int32_t>(t_stored * SE_ROW),
-      0x00020000);
-  auto dma = [&](int j, int c0, uint8_t* kd, uint8_t* vd) {
-    const int slot = lane & 15;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int r0 = 4 * wave + 16 * i;
-      const int row = r0 + (lane >> 4);
-      const int32_t off = (start_l[j] + c0 + row) * SE_ROW;
-      lds_dma16(k_rsrc, kd + r0 * SE_ROW, off + ((slot ^ (row & 15)) << 4));
-      if (MODE == 0) lds_dma16(v_rsrc, vd + r0 * SE_ROW, off + (slot << 4));
-    }
+  const int32_t run_start = static_cast<int32_t>(min(before + upto - own, t_stored));
+  const int32_t run_len = static_cast<int32_t>(min(before + upto, t_stored)) - run_start;
+  if (wave == 0 && lane < SE_CPW) len_l[lane] = run_len;  // read behind the last barrier
+  const uint32_t filled = static_cast<uint32_t>(__ballot(lane < ncl && run_len > 0));
+  struct Walk {
+    int j, c0, len, start;  // cluster, first token of the chunk in it, its run
   };
-  constexpr int DMA_PER_CHUNK = MODE == 0 ? 4 : 2;  // per wave
-  // |v_t|^2 and v_t . vc of chunk (j, c0) from V tile b into vn2_l / cdv_l[p]: token tid / 8,
-  // dims 16 (tid % 8) .. + 15, reduced over the token's 8 lanes
-  auto vstats = [&](int j, const uint8_t* vt, int p) {
-    const int pt = tid >> 3, pp = 2 * (tid & 7);
-    const uint8_t* vr = vt + pt * SE_ROW + pp * 16;
-    const float* cc = vc_l[j] + 8 * pp;
-    float pn = 0.0f, pc = 0.0f;
+  auto enter = [&](Walk& w, int from) {  // the first cluster with tokens at or after `from`; j = SE_CPW if none
+    const uint32_t rest = filled & ~((1u << from) - 1u);
+    w.j = rest != 0 ? __builtin_ctz(rest) : SE_CPW;
+    w.c0 = 0;
+    w.len = __builtin_amdgcn_readlane(run_len, w.j % SE_CPW);
+    w.start = __builtin_amdgcn_readlane(run_start, w.j % SE_CPW);
+  };
+  auto advance = [&](Walk& w) {
+    w.c0 += SE_CHUNK;
+    if (w.c0 >= w.len) enter(w, w.j + 1);
+  };
+  auto inside = [](const Walk& w) { return w.j < SE_CPW; };
+
+  // ---- K/V chunks land in LDS by DMA: 32 token rows of 256 bytes per tile; waves 0 .. 3 move
+  // rows 4 w .. 4 w + 3 and 16 + 4 w .. + 3 (1 KB per instruction).  The lane that fills slot p
+  // of row t fetches piece p ^ (t % 16) (the swizzle of the MFMA reads).  Rows past the
+  // cluster's run hold the next cluster's tokens (masked in the scores); rows past the stored
+  // tokens read as zero (buffer bounds).
+  const spr::i32x4_s k_desc = spr::buffer_desc(ks + kh * t_stored * SE_D, static_cast<int32_t>(t_stored * SE_ROW));
+  const spr::i32x4_s v_desc =
+      spr::buffer_desc(MODE == 0 ? vs + kh * t_stored * SE_D : ks, static_cast<int32_t>(t_stored * SE_ROW));
+  auto dma = [&](const Walk& w, int kt, int vt) {
+    if (wave < 4) {
+      const int slot = lane & 15;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const u32x4 v4 = *reinterpret_cast<const u32x4*>(vr + 16 * i);
-      const uint32_t w[4] = {v4.x, v4.y, v4.z, v4.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float lo = spr::bf16_lo(w[e]), hi = spr::bf16_hi(w[e]);
-        pn = __builtin_fmaf(lo, lo, pn);
-        pn = __builtin_fmaf(hi, hi, pn);
-        pc = __builtin_fmaf(lo, cc[8 * i + 2 * e], pc);
-        pc = __builtin_fmaf(hi, cc[8 * i + 2 * e + 1], pc);
+      for (int i = 0; i < 2; ++i) {
+        const int r0 = 4 * wave + 16 * i;
+        const int row = r0 + (lane >> 4);
+        const int32_t off = (w.start + w.c0 + row) * SE_ROW + ((slot ^ (row & 15)) << 4);
+        spr::lds_dma16(k_desc, k_tiles + kt + r0 * SE_ROW, off);
+        if (MODE == 0) spr::lds_dma16(v_desc, v_tiles + vt + r0 * SE_ROW, off);
       }
     }
-    pn = oct_sum(pn);
-    pc = oct_sum(pc);
-    if ((tid & 7) == 0) {
-      vn2_l[p][pt] = pn;
-      cdv_l[p][pt] = pc;
-    }
   };
-  // next (cluster, chunk) of the walk; j = ncl when done
-  auto advance = [&](int& j, int& c0) {
-    c0 += SE_CHUNK;
-    if (c0 >= cl_len(j)) {
-      c0 = 0;
-      j = nxt_l[j];
+  constexpr int DMA_PER_CHUNK = MODE == 0 ? 4 : 2;  // per wave that moves any
+
+  const int f_x = col & 15;
+  auto tile_frag = [&](const uint8_t* t, int s) {  // token row col, dims 16 s + 8 half + 0 .. 7
+    return *reinterpret_cast<const u32x4*>(t + col * SE_ROW + (((2 * s + half) ^ f_x) << 4));
+  };
+  // |v_t|^2 (the diagonal of V V^T) and -2 v_t . vc (V against the three pieces of vc in
+  // columns 0 .. 2) of a chunk: exact products, fp32 sums
+  auto vstats = [&](int j, const uint8_t* vt, int buf) {
+    f32x16 vv = f32x16{}, vc = f32x16{};
+    const uint16_t* brow = vc_l[col < 3 ? 3 * j + col : 3 * SE_CPW] + 8 * half;
+#pragma unroll
+    for (int s = 0; s < SE_KSTEPS; ++s) {
+      const u32x4 a = tile_frag(vt, s);
+      const u32x4 b = *reinterpret_cast<const u32x4*>(brow + 16 * s);
+      vv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(spr::as_bf16x8(a), spr::as_bf16x8(a), vv, 0, 0, 0);
+      vc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(spr::as_bf16x8(a), spr::as_bf16x8(b), vc, 0, 0, 0);
+    }
+    float diag = 0.0f;  // row col is element 4 (col / 8) + col % 4 of the half with bit 2 of col
+#pragma unroll
+    for (int e = 0; e < 16; ++e) diag = e == 4 * (col >> 3) + (col & 3) ? vv[e] : diag;
+    if (half == ((col >> 2) & 1)) vn_l[buf][col] = diag;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f32x4 c;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float x = vc[4 * i + r];  // columns 0 .. 3 (the last is zero) lie in one quad
+        x += dpp_mov<0xB1>(x);
+        x += dpp_mov<0x4E>(x);
+        c[r] = -2.0f * x;
+      }
+      if (col == 0) *reinterpret_cast<f32x4*>(&cd_l[buf][8 * i + 4 * half]) = c;
     }
   };
 
-  for (int q0 = 0; q0 < qn; q0 += 32 * SE_WAVES) {
-    const int q = q0 + 32 * wave + col;
-    const bool q_live = q < qn;
-    const bool wave_live = q0 + 32 * wave < qn;
-    const float* qrow = qc + (qh * qn + (q_live ? q : 0)) * SE_D;
-
-    // B fragments: q~ dims 16 s + 8 half + 0..7 as bf16 hi and lo
+  Walk wc, wn, wd;  // the next chunk to fold, to take statistics of, to DMA
+  enter(wc, 0);
+  wn = wd = wc;
+  int folded = 0, taken = 0, issued = 0;  // how many of each so far
+  // Step p folds chunks 2 p and 2 p + 1 and takes the statistics of the two after them; two more
+  // are in flight and another two go to the tiles of the step before.  Two chunks to a barrier
+  // let the waves of a SIMD drift apart, one's MFMAs beside another's exponentials.  Every wave
+  // takes the same steps.
+  auto issue = [&] {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (inside(wd)) {
+        dma(wd, issued % SE_TILES * SE_TILE, issued % SE_VTILES * SE_TILE);
+        ++issued;
+        advance(wd);
+      }
+    }
+  };
+  auto landed = [&](int upto) {  // chunks below `upto`, for every wave; two more may be in flight
+    if (issued >= upto + 2) spr::wait_vm<2 * DMA_PER_CHUNK>();
+    else if (issued == upto + 1) spr::wait_vm<DMA_PER_CHUNK>();
+    else spr::wait_vm<0>();
+    spr::lds_barrier();
+  };
+  auto first = [&] {
+    issue();
+    issue();
+    landed(2);
+    issue();
+  };
+  auto begin_step = [&] {
+    landed(folded + 4);
+    issue();
+  };
+  if (q_wave) {
+    // B fragments: q~ dims 16 s + 8 half + 0..7 as bf16 hi and lo, in registers before the
+    // first DMA (a later wait for them would drain it)
     u32x4 qhi[SE_KSTEPS], qlo[SE_KSTEPS];
 #pragma unroll
     for (int s = 0; s < SE_KSTEPS; ++s) {
-      float v[8];
-      if (q_live) {
-        const float4 a = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half);
-        const float4 b = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * half + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = 0.0f;
-      }
+      const float4 a = qraw[2 * s], b = qraw[2 * s + 1];
+      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
       uint32_t h[4], l[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -355,181 +419,152 @@ __global__ __launch_bounds__(SE_THREADS) void svg_ear_score_kernel(
       }
       qhi[s] = u32x4{h[0], h[1], h[2], h[3]};
       qlo[s] = u32x4{l[0], l[1], l[2], l[3]};
+      asm volatile("" : "+v"(qhi[s].x), "+v"(qhi[s].y), "+v"(qhi[s].z), "+v"(qhi[s].w));
+      asm volatile("" : "+v"(qlo[s].x), "+v"(qlo[s].y), "+v"(qlo[s].z), "+v"(qlo[s].w));
     }
-    // every wave is done with the previous query group (its tiles, statistics and cl_l)
-    __syncthreads();
-    if (MODE == 0) {
-      // centroid logits of this query group (written by svg_ear_centroid_logit_kernel)
-      for (int i = tid; i < SE_CPW * 32 * SE_WAVES; i += SE_THREADS) {
-        const int j = i / (32 * SE_WAVES), r = q0 + i % (32 * SE_WAVES);
-        cl_l[j][i % (32 * SE_WAVES)] = (j < ncl && r < qn) ? scores[(qh * qn + r) * kn + c_begin + j] : 0.0f;
-      }
-      __syncthreads();  // every wave has read l_c before any score of the group is written
-    }
-
-    float m = 0.0f, cw = 1.0f, esum = 0.0f;
-    int j = j_first, c0 = 0;       // chunk computed
-    int jv = j_first, cv = 0;      // chunk whose V statistics come next
-    int jd = j_first, cd = 0;      // next chunk to DMA
-    int issued = 0, step = 0;      // chunks DMA'd / computed in this query group
-    // chunks 0 .. 2 into tiles 0 .. 2 (named arrays, as in the loop)
-    auto prologue_dma = [&](uint8_t* kd, uint8_t* vd) {
-      if (jd < ncl) {
-        dma(jd, cd, kd, vd);
-        ++issued;
-        advance(jd, cd);
-      }
-    };
-    prologue_dma(k_l0, v_l0);
-    prologue_dma(k_l1, v_l1);
-    prologue_dma(k_l2, v_l2);
-    // chunk 0 landed (this wave's DMA), then every wave's; its V statistics
-    if (issued == 3) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DMA_PER_CHUNK) : "memory");
-    } else if (issued == 2) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA_PER_CHUNK) : "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    lds_barrier();
-    if (MODE == 0) vstats(jv, v_l0, 0);
-    advance(jv, cv);
-    // S^T of the chunk in tile kt: 16 MFMAs (hi and lo halves of q~ per 16-dim step)
     auto smma = [&](f32x16& acc, const uint8_t* kt) {
       acc = f32x16{};
 #pragma unroll
       for (int s = 0; s < SE_KSTEPS; ++s) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(kt + col * SE_ROW + (((2 * s + half) ^ (col & 15)) << 4));
+        const u32x4 a = tile_frag(kt, s);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(spr::as_bf16x8(a), spr::as_bf16x8(qhi[s]), acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(spr::as_bf16x8(a), spr::as_bf16x8(qlo[s]), acc, 0, 0, 0);
       }
     };
-    f32x16 acc_a, acc_b;
-    if (wave_live) smma(acc_a, k_l0);
-    // One chunk step s: DMAs chunk s + 3 into kd / vd, takes the V statistics of chunk
-    // s + 1 from vt1 into buf ^ 1, issues the MFMAs of chunk s + 1 (tile kt1) into
-    // acc_next and folds chunk s (acc_cur, statistics buf) into the running state: the
-    // matrix unit works on s + 1 while the VALU works on s.  Returns false when the walk
-    // is done.
-    auto chunk_step = [&](const uint8_t* kt1, const uint8_t* vt1, uint8_t* kd, uint8_t* vd, const int buf,
-                          f32x16& acc_cur, f32x16& acc_next) {
-      if (j >= ncl) return false;
-      const int cn = min(SE_CHUNK, cl_len(j) - c0);
-      const int jc = j;
-      const bool first = c0 == 0;
-      const bool last = c0 + SE_CHUNK >= cl_len(j);
-      // chunk step + 1 landed (this wave's DMA; the one of step + 2 may still be in flight),
-      // then every wave's; every wave is past step - 1, so its tiles and statistics are free
-      if (issued > step + 2) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA_PER_CHUNK) : "memory");
+    float ref = 0.0f, lc = 0.0f, top = 0.0f, esum = 0.0f, cw = 1.0f;
+    // S^T of a chunk (16 MFMAs), folded into the state:
+    // E = sum_t max(c_w^2 |vc|^2 + r (r |v|^2 - 2 c_w v.vc), 0) with r = e^(l_t - ref),
+    // c_w = e^(l_c - ref).  ref starts at l_c (c_w = 1: no product per element) and moves only
+    // when a logit passes it by SE_SLACK; the result does not depend on it but for rounding.
+    auto fold = [&](auto masked, const uint8_t* kt, int buf, int cn, int jc) {
+      constexpr bool MASKED = decltype(masked)::value;
+      f32x16 cur;
+      smma(cur, kt);
+      // element e is token 8 (e / 4) + 4 half + e % 4 of the chunk; a token past the run (the next
+      // cluster's, or zeros) gets the logit -inf, and its error term is cleared
+      const int lim = cn - 4 * half;
+      if (MASKED) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) cur[e] = 8 * (e / 4) + (e % 4) < lim ? cur[e] : -__builtin_huge_valf();
+      }
+      float cmax = -__builtin_huge_valf();
+#pragma unroll
+      for (int e = 0; e < 16; ++e) cmax = fmaxf(cmax, cur[e]);
+      // max over the raw dot products, scaled once: fl(a s) is monotone in a for s > 0
+      cmax = max_xor32(cmax) * scale;
+      top = fmaxf(top, cmax);
+      const bool up = cmax > ref + SE_SLACK;
+      if (__ballot(up) != 0ull) {
+        const float to = up ? cmax : ref;
+        const float alpha = up ? exp_fast(ref - to) : 1.0f;
+        esum *= MODE == 0 ? alpha * alpha : alpha;
+        ref = to;
+        cw = up ? exp_fast(lc - ref) : cw;
+      }
+      const float c1 = scale * SE_LOG2E;
+      const float negm = -ref * SE_LOG2E;
+      float add0 = 0.0f, add1 = 0.0f;
+      auto terms = [&](auto scaled) {
+        constexpr bool SCALED = decltype(scaled)::value;
+        const float base = SCALED ? cw * cw * vc2_l[jc] : vc2_l[jc];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const f32x4 vn = *reinterpret_cast<const f32x4*>(&vn_l[buf][8 * i + 4 * half]);
+          const f32x4 cd = *reinterpret_cast<const f32x4*>(&cd_l[buf][8 * i + 4 * half]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(cur[4 * i + r], c1, negm));
+            float err = fmaxf(__builtin_fmaf(w, __builtin_fmaf(w, vn[r], SCALED ? cw * cd[r] : cd[r]), base), 0.0f);
+            if (MASKED) err = 8 * i + r < lim ? err : 0.0f;
+            if (r % 2 == 0) add0 += err; else add1 += err;
+          }
+        }
+      };
+      if (MODE == 0) {
+        if (__ballot(cw != 1.0f) == 0ull) terms(std::false_type{}); else terms(std::true_type{});
       } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
-      lds_barrier();
-      if (jd < ncl) {
-        dma(jd, cd, kd, vd);
-        ++issued;
-        advance(jd, cd);
-      }
-      const bool has_next = jv < ncl;
-      if (has_next) {
-        if (MODE == 0) vstats(jv, vt1, buf ^ 1);
-        advance(jv, cv);
-      }
-      advance(j, c0);
-      ++step;
-      if (wave_live) {
-        if (has_next) smma(acc_next, kt1);
-        if (first) {
-          m = MODE == 0 ? cl_l[jc][32 * wave + col] : -__builtin_huge_valf();
-          cw = 1.0f;
-          esum = 0.0f;
-        }
-        f32x16* acc = &acc_cur;
-        constexpr int NB = 1;
-        // element e of block b is token 32 b + 8 (e / 4) + 4 half + e % 4 of the chunk
-        // The chunk's 16 elements per lane, straight-line.  A full chunk (the common case)
-        // needs no mask; in a partial one a token past the end (its rows hold the next
-        // cluster's tokens or zeros) gets exponent -inf (weight 0) and its error term is
-        // cleared bitwise, so no value of those rows reaches the sums.
-        auto update = [&](auto masked) {
-          constexpr bool MASKED = decltype(masked)::value;
-          auto live = [&](int b, int e) { return 32 * b + 8 * (e / 4) + 4 * half + (e % 4) < cn; };
-          // max over the raw dot products, scaled once: fl(a s) is monotone in a for s > 0,
-          // so this is the max of the scaled logits
-          float cmax = -__builtin_huge_valf();
 #pragma unroll
-          for (int b = 0; b < NB; ++b) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) cmax = fmaxf(cmax, (!MASKED || live(b, e)) ? acc[b][e] : -__builtin_huge_valf());
-          }
-          cmax = max_xor32(cmax) * scale;
-          const float m_new = fmaxf(m, cmax);
-          const float alpha = exp_fast(m - m_new);
-          // e^(l - m_new) = 2^(dot * scale * log2 e - m_new * log2 e), one fma per element
-          const float c1 = scale * SE_LOG2E;
-          const float negm = -m_new * SE_LOG2E;
-          float add = 0.0f;
-          if (MODE == 0) {
-            cw *= alpha;
-            esum *= alpha * alpha;
-            const float base = cw * cw * vc2_l[jc];
-            const float two_cw = 2.0f * cw;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const int t0 = 32 * b + 8 * i + 4 * half;
-                const float4 vn = *reinterpret_cast<const float4*>(&vn2_l[buf][t0]);
-                const float4 cd = *reinterpret_cast<const float4*>(&cdv_l[buf][t0]);
-                const float vna[4] = {vn.x, vn.y, vn.z, vn.w};
-                const float cda[4] = {cd.x, cd.y, cd.z, cd.w};
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                  const bool lv = !MASKED || live(b, 4 * i + r);
-                  const float x = __builtin_fmaf(acc[b][4 * i + r], c1, negm);
-                  const float tw = __builtin_amdgcn_exp2f(lv ? x : -__builtin_huge_valf());
-                  // w_c^2 |vc|^2 + w_t (w_t |v|^2 - 2 w_c v.vc)
-                  const float err =
-                      fmaxf(__builtin_fmaf(tw, __builtin_fmaf(tw, vna[r], -two_cw * cda[r]), base), 0.0f);
-                  add += MASKED ? __int_as_float(__float_as_int(err) & -static_cast<int>(lv)) : err;
-                }
-              }
-            }
-          } else {
-            esum *= alpha;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-#pragma unroll
-              for (int e = 0; e < 16; ++e) {
-                const bool lv = !MASKED || live(b, e);
-                add += __builtin_amdgcn_exp2f(lv ? __builtin_fmaf(acc[b][e], c1, negm) : -__builtin_huge_valf());
-              }
-            }
-          }
-          esum += add;
-          m = m_new;
-        };
-        if (cn == SE_CHUNK) {
-          update(std::false_type{});
-        } else {
-          update(std::true_type{});
-        }
-        if (last) {
-          const float total = sum_xor32(esum);
-          if (q_live && half == 0) {
-            const float score = MODE == 0
-                                    ? logf(fmaxf(total / static_cast<float>(cl_len(jc)), 1.0e-30f)) + 2.0f * m
-                                    : logf(fmaxf(total, 1.0e-30f)) + m;
-            scores[(qh * qn + q) * kn + c_begin + jc] = score;
-          }
+        for (int e = 0; e < 16; e += 2) {
+          add0 += __builtin_amdgcn_exp2f(__builtin_fmaf(cur[e], c1, negm));
+          add1 += __builtin_amdgcn_exp2f(__builtin_fmaf(cur[e + 1], c1, negm));
         }
       }
-      return true;
+      esum += add0 + add1;
     };
-    while (chunk_step(k_l1, v_l1, k_l3, v_l3, 0, acc_a, acc_b) && chunk_step(k_l2, v_l2, k_l0, v_l0, 1, acc_b, acc_a) &&
-           chunk_step(k_l3, v_l3, k_l1, v_l1, 0, acc_a, acc_b) && chunk_step(k_l0, v_l0, k_l2, v_l2, 1, acc_b, acc_a)) {
+    if (inside(wc)) first();
+    while (inside(wc)) {
+      begin_step();
+      for (int i = 0; i < 2 && inside(wc); ++i) {
+        if (sets == 1 || i == set) {
+          const int slot = set * rows + 32 * (wave % qwaves) + col;
+          if (wc.c0 < sets * SE_CHUNK) {  // this wave's first chunk of the cluster
+            lc = rf_l[wc.j][slot];
+            ref = lc;
+            top = lc;
+            cw = 1.0f;
+            esum = 0.0f;
+          }
+          const int cn = min(SE_CHUNK, wc.len - wc.c0);
+          const uint8_t* kt = k_tiles + folded % SE_TILES * SE_TILE;
+          if (cn == SE_CHUNK) fold(std::false_type{}, kt, folded & 3, cn, wc.j);
+          else fold(std::true_type{}, kt, folded & 3, cn, wc.j);
+          if (wc.c0 + sets * SE_CHUNK >= wc.len) {  // its last
+            const float total = sum_xor32(esum);
+            if (half == 0) {
+              es_l[wc.j][slot] = total;
+              rf_l[wc.j][slot] = ref;
+              tp_l[wc.j][slot] = top;
+            }
+          }
+        }
+        ++folded;
+        advance(wc);
+      }
     }
+  } else {
+    auto stats = [&] {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (inside(wn)) {
+          if (i == stat) vstats(wn.j, v_tiles + taken % SE_VTILES * SE_TILE, taken & 3);
+          ++taken;
+          advance(wn);
+        }
+      }
+    };
+    if (inside(wc)) {
+      first();
+      stats();
+    }
+    while (inside(wc)) {
+      begin_step();
+      stats();
+      for (int i = 0; i < 2 && inside(wc); ++i) {
+        ++folded;
+        advance(wc);
+      }
+    }
+  }
+  __syncthreads();
+  // scores out, SE_CPW consecutive clusters of a query row at a time; empty clusters -inf
+  for (int i = tid; i < SE_CPW * rows; i += nthr) {
+    const int j = i % SE_CPW, r = i / SE_CPW;
+    if (j >= ncl || q0 + r >= qn) continue;
+    float total = es_l[j][r], ref = rf_l[j][r], top = tp_l[j][r];
+    if (sets == 2) {
+      const float r1 = rf_l[j][rows + r], to = fmaxf(ref, r1);
+      const float a0 = ref == to ? 1.0f : exp_fast(ref - to), a1 = r1 == to ? 1.0f : exp_fast(r1 - to);
+      total = MODE == 0 ? total * (a0 * a0) + es_l[j][rows + r] * (a1 * a1) : total * a0 + es_l[j][rows + r] * a1;
+      ref = to;
+      top = fmaxf(top, tp_l[j][rows + r]);
+    }
+    float score = -__builtin_huge_valf();
+    if ((filled >> j) & 1u) {
+      // value error: log(max(E / n, 1e-30)) of the weights taken from the largest logit
+      score = MODE == 0 ? fmaxf(logf(total / static_cast<float>(len_l[j])) + 2.0f * ref, -69.07755278982137f + 2.0f * top)
+                        : logf(fmaxf(total, 1.0e-30f)) + ref;
+    }
+    scores[(qh * qn + q0 + r) * kn + c_begin + j] = score;
   }
 }
 
@@ -732,7 +767,17 @@ extern "C" int spr_svg_ear_scores(const float* q_centroids, const uint16_t* k_so
     SPR_REQUIRE(!(jensen_var_cap > 0.0f) || var_k_diag != nullptr,
                 "spr_svg_ear_scores: Jensen-aware routing requires var_k_diag");
   }
-  const dim3 grid(static_cast<uint32_t>((kn + SE_CPW - 1) / SE_CPW), static_cast<uint32_t>(q_heads));
+  // Query blocks of 32 rows, one wave each, in groups of equal size of at most SE_QWAVES; up to
+  // five blocks get two waves each.  One more wave takes the V statistics, and four move the tiles.
+  const int32_t qblocks = (qn + 31) / 32;
+  const int32_t qgroups = (qblocks + SE_QWAVES - 1) / SE_QWAVES;
+  const int32_t qwaves = (qblocks + qgroups - 1) / qgroups;
+  const int32_t sets = 2 * qwaves <= SE_QWAVES ? 2 : 1;
+  const int64_t turns = static_cast<int64_t>((kn + 8 * SE_CPW - 1) / (8 * SE_CPW)) * qgroups;
+  SPR_REQUIRE(turns * 8 < (int64_t(1) << 31), "spr_svg_ear_scores: grid too large");
+  const dim3 grid(static_cast<uint32_t>(turns * 8), static_cast<uint32_t>(q_heads));
+  const int32_t waves = qwaves * sets + (mode == 0 ? SE_SWAVES : 0);
+  const uint32_t threads = 64 * (waves < 4 ? 4 : waves);
   if (mode == 0) {
     const bool jensen = jensen_var_cap > 0.0f;
     svg_ear_centroid_logit_kernel<<<dim3(static_cast<uint32_t>((kn + CL_CLUSTERS - 1) / CL_CLUSTERS),
@@ -741,12 +786,12 @@ extern "C" int spr_svg_ear_scores(const float* q_centroids, const uint16_t* k_so
                                     SE_THREADS, 0, stream>>>(q_centroids, k_centroids, jensen ? var_k_diag : nullptr,
                                                              jensen ? jensen_var_cap : 0.0f, qn, kn, group, scores);
     SPR_LAUNCHED("svg_ear_centroid_logit_kernel");
-    svg_ear_score_kernel<0><<<grid, SE_THREADS, 0, stream>>>(q_centroids, k_sorted, v_sorted, v_centroids, k_sizes,
-                                                             qn, kn, t_stored, group, scores);
+    svg_ear_score_kernel<0><<<grid, threads, 0, stream>>>(q_centroids, k_sorted, v_sorted, v_centroids, k_sizes, qn,
+                                                          kn, t_stored, group, qgroups, qwaves, sets, scores);
     SPR_LAUNCHED("svg_ear_score_kernel<value>");
   } else {
-    svg_ear_score_kernel<1><<<grid, SE_THREADS, 0, stream>>>(q_centroids, k_sorted, nullptr, nullptr, k_sizes, qn,
-                                                             kn, t_stored, group, scores);
+    svg_ear_score_kernel<1><<<grid, threads, 0, stream>>>(q_centroids, k_sorted, nullptr, nullptr, k_sizes, qn, kn,
+                                                          t_stored, group, qgroups, qwaves, sets, scores);
     SPR_LAUNCHED("svg_ear_score_kernel<mass>");
   }
   return SPR_OK;

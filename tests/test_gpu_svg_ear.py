@@ -86,6 +86,30 @@ def test_attention_mass_scores_match_oracle(dev, oracle, qh, group, qn, si):
     _check(got, oracle.attention_mass_scores(qc, k, sizes, group))
 
 
+@pytest.mark.parametrize("qn", [1, 33, 160, 161, 320, 321])  # two waves per block; one; two groups
+@pytest.mark.parametrize("kn,qscale", [(7, 0.4), (65, 0.4), (9, 6.0)])
+def test_scores_at_the_edges_of_the_wave_split(dev, oracle, qn, kn, qscale):
+    """Query blocks at each way they are shared out, cluster groups of eight and a remainder,
+    runs around one, two and three chunks; at qscale 6 logits pass the centroid's by far more
+    than the reference moves for.  Scores reach several hundred there, so the bound is 2e-3 and
+    1e-5 of the score (its fp32 rounding times a few)."""
+    from sparsepr_amd.kernels.svg_ear import attention_mass_scores_triton, svg_ear_value_error_scores_triton
+
+    sizes = np.resize(np.array([0, 33, 1, 64, 96, 65, 32, 31, 2], np.int32), (2, kn))
+    qc, k, v, kc, vc, _ = _case(qn + kn, 2, 1, qn, sizes, qscale=qscale)
+    k, v = _bf16_np(oracle, k), _bf16_np(oracle, v)
+    dk, dv, dq, ds = to_dev(k, dev, torch.bfloat16), to_dev(v, dev, torch.bfloat16), to_dev(qc, dev), to_dev(sizes, dev)
+    got = svg_ear_value_error_scores_triton(qcentroids=dq, k_sorted=dk, v_sorted=dv, kcentroids=to_dev(kc, dev),
+                                            vcentroids=to_dev(vc, dev), kcluster_sizes=ds, gqa_group=1)
+    mass = attention_mass_scores_triton(qcentroids=dq, k_sorted=dk, kcluster_sizes=ds, gqa_group=1)
+    for a, ref in ((got, oracle.svg_ear_value_error_scores(qc, k, v, kc, vc, sizes, 1)),
+                   (mass, oracle.attention_mass_scores(qc, k, sizes, 1))):
+        a = a.cpu().numpy().astype(np.float64)
+        fin = np.isfinite(ref)
+        assert (np.isneginf(a) == ~fin).all()
+        assert (np.abs(a[fin] - ref[fin]) <= ATOL + 1e-5 * np.abs(ref[fin])).all()
+
+
 def test_grouped_scores_equal_ungrouped(dev, oracle):
     from sparsepr_amd.kernels.svg_ear import (svg_ear_grouped_value_error_scores_triton,
                                               svg_ear_value_error_scores_triton)
