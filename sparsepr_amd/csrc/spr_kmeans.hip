@@ -998,6 +998,10 @@ __device__ void finalize_mean(double s, int32_t count, int64_t b, int32_t cl, in
 // 118,800 rows; slices sized from the average left it to two workgroups: 204 us per update
 // against 134 us on uniform labels).
 constexpr int MEAN_SLICE = 512;
+// Up to this many points per batch one workgroup takes a whole cluster, with neither plan nor
+// finalize launch: 24 x 8,192 x 64 (128 clusters) 21 us in three launches, 15.5 in one (both with
+// 8 us of graph replay); with a seventh of the points in one cluster 24.5 and 28.
+constexpr int64_t MEAN_WHOLE_N = 8192;
 
 // One workgroup per batch: slice_base[b][c] = the first slice of cluster c (exclusive scan of
 // ceil(rows_c / MEAN_SLICE), c = 0 .. k; capped at maxs, the slices the workspace holds, so
@@ -1057,7 +1061,7 @@ __global__ __launch_bounds__(256) void mean_slice_plan_kernel(const int32_t* __r
 }
 
 // T: uint16_t (bf16) or float.  Workgroup (s, b) sums slice s of batch b (rows
-// slice_rows[b][s] of the sorted order) in fp64.  The one slice of a cluster finalizes its
+// slice_rows[b][s] of the sorted order; without a plan, cluster s) in fp64.  The one slice of a cluster finalizes its
 // mean directly; otherwise the sum goes to partial[b][s][D], and
 // centroid_mean_finalize_kernel adds the cluster's slices in order (the result does not
 // depend on the split).
@@ -1082,8 +1086,14 @@ __global__ __launch_bounds__(256) void centroid_mean_kernel(
   const int rg = tid / VPR;
   const int64_t b = blockIdx.y;
   const int32_t n32 = static_cast<int32_t>(n);
-  const int4 rr = slice_rows[b * maxs + blockIdx.x];
-  if (rr.w == 0) return;  // past the last slice
+  int4 rr;
+  if (slice_rows != nullptr) {
+    rr = slice_rows[b * maxs + blockIdx.x];
+    if (rr.w == 0) return;  // past the last slice
+  } else {  // short inputs: a whole cluster, empty ones included
+    const int32_t c = static_cast<int32_t>(blockIdx.x);
+    rr = int4{offsets[b * (k + 1) + c], offsets[b * (k + 1) + c + 1], c, 1};
+  }
   // the plan's ranges lie in [0, n); clamp anyway
   const int32_t start = min(max(rr.x, 0), n32);
   const int32_t end = min(max(rr.y, start), n32);
@@ -1589,6 +1599,7 @@ extern "C" int spr_centroid_mean(const void* x, int32_t dtype, const int32_t* so
   SPR_REQUIRE(sorted_idx && offsets && old, "spr_centroid_mean: null pointer");
   SPR_REQUIRE(n == 0 || x, "spr_centroid_mean: null x");
   SPR_REQUIRE(n < (int64_t(1) << 31), "spr_centroid_mean: n too large");
+  const bool sliced = n > MEAN_WHOLE_N;
   const int64_t maxs = mean_max_slices(n, k);
   SPR_REQUIRE(maxs < (int64_t(1) << 31), "spr_centroid_mean: too many clusters");
   const size_t need = spr_centroid_mean_workspace(batch, n, k, d);
@@ -1603,17 +1614,21 @@ extern "C" int spr_centroid_mean(const void* x, int32_t dtype, const int32_t* so
   ws += align16(static_cast<size_t>(batch * (k + 1)) * sizeof(int32_t));
   int4* slice_rows = reinterpret_cast<int4*>(ws);
   const int32_t ms = static_cast<int32_t>(maxs);
-  mean_slice_plan_kernel<<<dim3(static_cast<uint32_t>(batch)), 256, 0, stream>>>(offsets, n, k, ms, slice_base,
-                                                                                 slice_rows);
-  SPR_LAUNCHED("mean_slice_plan_kernel");
-  dim3 grid(static_cast<uint32_t>(maxs), static_cast<uint32_t>(batch));
+  if (sliced) {
+    mean_slice_plan_kernel<<<dim3(static_cast<uint32_t>(batch)), 256, 0, stream>>>(offsets, n, k, ms, slice_base,
+                                                                                   slice_rows);
+    SPR_LAUNCHED("mean_slice_plan_kernel");
+  } else {
+    slice_rows = nullptr;
+  }
+  dim3 grid(static_cast<uint32_t>(sliced ? maxs : k), static_cast<uint32_t>(batch));
   dim3 fgrid(static_cast<uint32_t>(k), static_cast<uint32_t>(batch));
 #define SPR_MEAN_CASE(T, DD)                                                                                 \
   do {                                                                                                       \
     centroid_mean_kernel<T, DD><<<grid, 256, 0, stream>>>(                                                   \
         static_cast<const T*>(x), sorted_idx, slice_rows, n, ms, partial, offsets, static_cast<const T*>(old), k, \
         mean32, static_cast<T*>(out), shift_max, sums_accum, counts_accum, c_sq_out);                         \
-    centroid_mean_finalize_kernel<T, DD><<<fgrid, 256, 0, stream>>>(                                         \
+    if (sliced) centroid_mean_finalize_kernel<T, DD><<<fgrid, 256, 0, stream>>>(                                         \
         partial, slice_base, ms, offsets, static_cast<const T*>(old), n, k, mean32, static_cast<T*>(out),    \
         shift_max, sums_accum, counts_accum, c_sq_out);                                                      \
   } while (0)

@@ -6,24 +6,34 @@
 // start offsets that the block-sparse attention schedule and the centroid
 // update consume.  Within a cluster tokens keep ascending index order.
 //
-// Three launches, all HBM/latency-light:
+// Rows of up to SMALL_N labels (and up to SMALL_BINS bins): one launch, one workgroup per row.
+// Longer rows, three launches:
 //   1. per (row, chunk of CHUNK tokens) label histogram in LDS;
 //   2. per row: label totals, exclusive scan over labels, per-chunk bases;
-//   3. per (row, chunk): one wave walks the chunk in order, ranks equal labels
-//      inside each 64-token group with readlane compares, scatters token ids.
+//   3. per (row, chunk): every wave ranks a consecutive part of the chunk against counters of
+//      its own, the counters become bases by a scan over the waves, and the token ids scatter.
+// What bounds them is the serial chain of a wave's 64-token groups (each ranks against the
+// counters the one before left, an LDS round trip), so a chunk is shared by as many waves as
+// the counters leave room for: 24 rows of 118,800 labels, 256 bins: 57 us (one wave per 1024
+// labels, 39 of them in the scatter) -> 44 us; 2 rows of 4096, 64 bins: 18 -> 6.4 us.
 // Labels outside [0, k) go to a trailing overflow bucket (sorted last).
+#include <type_traits>
+
 #include "spr_common.h"
 
 namespace {
 
-constexpr int CHUNK = 1024;
+constexpr int CHUNK = 4096;
 constexpr int MAX_BINS = 8192;  // k + 1 <= MAX_BINS (32 KB of LDS counters)
+constexpr int COUNTERS = 16384;   // LDS counters of a ranking workgroup (64 KB), shared by its waves
+constexpr int SMALL_N = 16384;    // longest row sorted by one workgroup of 16 waves ...
+constexpr int SMALL_BINS = COUNTERS / 16;  // ... whose counters fit
 
 __device__ __forceinline__ uint32_t bin_of(int32_t label, int32_t k) {
   return (label >= 0 && label < k) ? static_cast<uint32_t>(label) : static_cast<uint32_t>(k);
 }
 
-__global__ __launch_bounds__(256) void label_hist_kernel(const int32_t* __restrict__ labels, int64_t n,
+__global__ __launch_bounds__(512) void label_hist_kernel(const int32_t* __restrict__ labels, int64_t n,
                                                          int32_t k, int32_t nchunks,
                                                          int32_t* __restrict__ hist) {
   extern __shared__ int32_t h[];  // [k + 1]
@@ -116,56 +126,127 @@ __global__ __launch_bounds__(1024) void label_scan_kernel(int32_t* __restrict__ 
   }
 }
 
-// One wave per (row, chunk): ranks must follow token order, so the chunk is
-// walked in 64-token groups by a single wave.
-__global__ __launch_bounds__(64) void label_scatter_kernel(const int32_t* __restrict__ labels, int64_t n,
-                                                           int32_t k, int32_t nchunks,
-                                                           const int32_t* __restrict__ bases,
-                                                           int32_t* __restrict__ sorted_idx) {
-  extern __shared__ int32_t cnt[];  // [k + 1]
-  const int32_t bins = k + 1;
-  const int nbits = 32 - __builtin_clz(static_cast<uint32_t>(bins));  // 2^nbits > k + 1 > every bin
-  const int64_t row = blockIdx.y;
-  const int lane = threadIdx.x;
-  const int32_t* b = bases + (row * nchunks + blockIdx.x) * bins;
-  for (int j = lane; j < bins; j += 64) cnt[j] = b[j];
-  const int64_t c0 = static_cast<int64_t>(blockIdx.x) * CHUNK;
-  const int64_t c1 = c0 + CHUNK < n ? c0 + CHUNK : n;
-  // all of the chunk's labels are loaded before the first ranking step
-  constexpr int GROUPS = CHUNK / 64;
-  int32_t bins_of[GROUPS];
+// Ranks of a wave's labels among its earlier equal ones: group g of 64 consecutive labels sits
+// in bin[g] (-1 past the end), cnt holds the wave's count per bin, which the ranks extend.
+template <int G>
+__device__ __forceinline__ void rank_groups(const int32_t (&bin)[G], int32_t (&rank)[G], int nbits, int lane,
+                                            int32_t* __restrict__ cnt) {
 #pragma unroll
-  for (int i = 0; i < GROUPS; ++i) {
-    const int64_t t = c0 + i * 64 + lane;
-    bins_of[i] = t < c1 ? static_cast<int32_t>(bin_of(labels[row * n + t], k)) : -1;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < GROUPS; ++i) {
-    const int64_t g = c0 + i * 64;
-    if (g >= c1) break;
-    const int64_t t = g + lane;
-    const bool live = t < c1;
-    const int32_t bin = bins_of[i];
+  for (int g = 0; g < G; ++g) {
     // lanes holding the same bin, one ballot per bin bit (nbits bits hold every bin and
-    // keep the pattern of -1, past the chunk, apart from all of them); the rank is the
+    // keep the pattern of -1, past the end, apart from all of them); the rank is the
     // number of such lanes below this one, which keeps the sort stable
     uint64_t same = ~0ull;
     for (int bit = 0; bit < nbits; ++bit) {
-      const bool set = (bin >> bit) & 1;
+      const bool set = (bin[g] >> bit) & 1;
       const uint64_t m = __ballot(set);
       same &= set ? m : ~m;
     }
-    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    const int below = __popcll(same & ((1ull << lane) - 1ull));
     const int count = __popcll(same);
-    int32_t pos = 0;
-    if (live) pos = cnt[bin] + rank;
+    const bool live = bin[g] >= 0;
+    rank[g] = live ? cnt[bin[g]] + below : 0;
     __builtin_amdgcn_wave_barrier();
-    if (live) {
-      if (pos >= 0 && pos < n) sorted_idx[row * n + pos] = static_cast<int32_t>(t);
-      if (rank == count - 1) cnt[bin] += count;
+    if (live && below == count - 1) cnt[bin[g]] = rank[g] + 1;
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Workgroup per (row, chunk) of W waves; wave w ranks labels w * 64 G .. + 64 G of the chunk.
+template <int W>
+__global__ __launch_bounds__(W * 64) void label_scatter_kernel(const int32_t* __restrict__ labels, int64_t n,
+                                                               int32_t k, int32_t nchunks,
+                                                               const int32_t* __restrict__ bases,
+                                                               int32_t* __restrict__ sorted_idx) {
+  extern __shared__ int32_t cnt[];  // [W][k + 1]
+  constexpr int G = CHUNK / 64 / W;
+  const int32_t bins = k + 1;
+  const int nbits = 32 - __builtin_clz(static_cast<uint32_t>(bins));  // 2^nbits > k + 1 > every bin
+  const int64_t row = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * CHUNK + wave * (64 * G) + lane;
+  int32_t bin[G], rank[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int64_t t = t0 + 64 * g;
+    bin[g] = t < n ? static_cast<int32_t>(bin_of(labels[row * n + t], k)) : -1;
+  }
+  for (int j = tid; j < W * bins; j += W * 64) cnt[j] = 0;
+  __syncthreads();
+  rank_groups<G>(bin, rank, nbits, lane, cnt + wave * bins);
+  __syncthreads();
+  const int32_t* b = bases + (row * nchunks + blockIdx.x) * bins;
+  for (int j = tid; j < bins; j += W * 64) {
+    int32_t run = b[j];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const int32_t c = cnt[w * bins + j];
+      cnt[w * bins + j] = run;
+      run += c;
     }
-    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    if (bin[g] < 0) continue;
+    const int64_t pos = static_cast<int64_t>(cnt[wave * bins + bin[g]]) + rank[g];
+    if (pos >= 0 && pos < n) sorted_idx[row * n + pos] = static_cast<int32_t>(t0 + 64 * g);
+  }
+}
+
+// A whole row in one workgroup of 16 waves, 64 G labels each (n <= 1024 G): ranks, then the
+// counters' scan over waves and bins gives sizes, offsets and the waves' bases.
+template <int G>
+__global__ __launch_bounds__(1024) void label_sort_small_kernel(const int32_t* __restrict__ labels, int32_t n,
+                                                                int32_t k, int32_t* __restrict__ sorted_idx,
+                                                                int32_t* __restrict__ sizes,
+                                                                int32_t* __restrict__ offsets) {
+  extern __shared__ int32_t cnt[];  // [16][k + 1]
+  __shared__ int32_t wsum[16];
+  constexpr int W = 16;
+  const int32_t bins = k + 1;  // at most SMALL_BINS: one bin per thread below
+  const int nbits = 32 - __builtin_clz(static_cast<uint32_t>(bins));
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int32_t* lab = labels + row * n;
+  const int32_t t0 = wave * (64 * G) + lane;
+  int32_t bin[G], rank[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) bin[g] = t0 + 64 * g < n ? static_cast<int32_t>(bin_of(lab[t0 + 64 * g], k)) : -1;
+  for (int j = tid; j < W * bins; j += W * 64) cnt[j] = 0;
+  __syncthreads();
+  rank_groups<G>(bin, rank, nbits, lane, cnt + wave * bins);
+  __syncthreads();
+  int32_t total = 0;
+  if (tid < bins) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) total += cnt[w * bins + tid];
+  }
+  int32_t incl = total;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int32_t up = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += up;
+  }
+  if (lane == 63) wsum[wave] = incl;
+  __syncthreads();
+  int32_t run = incl - total;
+  for (int w = 0; w < wave; ++w) run += wsum[w];
+  if (tid < bins) {
+    if (sizes != nullptr && tid < k) sizes[row * k + tid] = total;
+    if (offsets != nullptr) offsets[row * (k + 1) + tid] = run;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const int32_t c = cnt[w * bins + tid];
+      cnt[w * bins + tid] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    if (bin[g] < 0) continue;
+    const int32_t pos = cnt[wave * bins + bin[g]] + rank[g];
+    if (pos >= 0 && pos < n) sorted_idx[row * n + pos] = t0 + 64 * g;
   }
 }
 
@@ -175,9 +256,14 @@ __global__ void fill_i32_kernel(int32_t* __restrict__ p, int64_t count, int32_t 
     p[i] = value;
 }
 
+// One launch instead of three; one workgroup per row is also the faster up to this length
+// (24 rows, 128 bins: 16,384 labels 20.7 us, 16,385 in three launches 22, their gaps aside).
+bool sorts_small(int64_t n, int32_t k) { return n <= SMALL_N && k + 1 <= SMALL_BINS; }
+
 }  // namespace
 
 extern "C" size_t spr_argsort_labels_workspace(int64_t rows, int64_t n, int32_t k) {
+  if (sorts_small(n, k)) return 16;  // none is used
   const int64_t nchunks = spr::ceil_div(n, CHUNK);
   return static_cast<size_t>(rows * nchunks * (static_cast<int64_t>(k) + 1) * 4);
 }
@@ -205,14 +291,33 @@ extern "C" int spr_argsort_labels(const int32_t* labels, int64_t rows, int64_t n
     spr_set_error("spr_argsort_labels: workspace %zu < %zu bytes", workspace_bytes, need);
     return SPR_EWORKSPACE;
   }
+  const size_t bin_bytes = static_cast<size_t>(k + 1) * sizeof(int32_t);
+  if (sorts_small(n, k)) {
+    if (n <= 4096) {
+      label_sort_small_kernel<4><<<dim3(rows), 1024, 16 * bin_bytes, stream>>>(labels, static_cast<int32_t>(n), k,
+                                                                              sorted_idx, sizes, offsets);
+    } else {
+      label_sort_small_kernel<16><<<dim3(rows), 1024, 16 * bin_bytes, stream>>>(labels, static_cast<int32_t>(n), k,
+                                                                               sorted_idx, sizes, offsets);
+    }
+    SPR_LAUNCHED("label_sort_small_kernel");
+    return SPR_OK;
+  }
   const int32_t nchunks = static_cast<int32_t>(spr::ceil_div(n, CHUNK));
   int32_t* hist = static_cast<int32_t*>(workspace);
-  const size_t bin_bytes = static_cast<size_t>(k + 1) * sizeof(int32_t);
-  label_hist_kernel<<<dim3(nchunks, rows), 256, bin_bytes, stream>>>(labels, n, k, nchunks, hist);
+  label_hist_kernel<<<dim3(nchunks, rows), 512, bin_bytes, stream>>>(labels, n, k, nchunks, hist);
   SPR_LAUNCHED("label_hist_kernel");
   label_scan_kernel<<<dim3(rows), 1024, 0, stream>>>(hist, k, nchunks, sizes, offsets);
   SPR_LAUNCHED("label_scan_kernel");
-  label_scatter_kernel<<<dim3(nchunks, rows), 64, bin_bytes, stream>>>(labels, n, k, nchunks, hist, sorted_idx);
+  auto scatter = [&](auto waves) {
+    constexpr int W = decltype(waves)::value;
+    label_scatter_kernel<W><<<dim3(nchunks, rows), W * 64, W * bin_bytes, stream>>>(labels, n, k, nchunks, hist,
+                                                                                    sorted_idx);
+  };
+  if (16 * (k + 1) <= COUNTERS) scatter(std::integral_constant<int, 16>{});
+  else if (8 * (k + 1) <= COUNTERS) scatter(std::integral_constant<int, 8>{});
+  else if (4 * (k + 1) <= COUNTERS) scatter(std::integral_constant<int, 4>{});
+  else scatter(std::integral_constant<int, 2>{});
   SPR_LAUNCHED("label_scatter_kernel");
   return SPR_OK;
 }

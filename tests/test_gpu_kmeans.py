@@ -116,6 +116,31 @@ def test_centroid_mean_skewed_clusters(dev, oracle, dtype, d):
     assert (res.sizes.cpu().numpy() == counts).all()
 
 
+@pytest.mark.parametrize("n", [1, 700, 8192, 8193])  # whole clusters per workgroup up to 8,192 points
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float32, 16)])
+def test_centroid_mean_of_short_inputs(dev, oracle, n, dtype, d):
+    """Means bit-exact to the float64 ones, empty clusters from the previous centroids, the norms
+    and the shift with them, on either side of the length that needs a slice plan."""
+    from sparsepr_amd.flash_kmeans.kmeans_impl import centroid_sq, centroid_update_sorted
+
+    rng = np.random.default_rng(n + d)
+    b, k = 3, 21
+    x = _gmm(oracle, rng, b, n, d, 9)
+    labels = rng.integers(2, k, (b, n)).astype(np.int32)
+    labels[rng.random((b, n)) < 0.5] = 1
+    old = oracle.to_bf16(rng.standard_normal((b, k, d)).astype(np.float32))
+    norms = torch.empty((b, k), device=dev)
+    res = centroid_update_sorted(to_dev(x, dev, dtype), to_dev(labels, dev), to_dev(old, dev, dtype),
+                                 want_mean32=True, want_shift=True, c_sq_out=norms)
+    cent, mean32, counts = oracle.centroid_update(x, labels, old, out_bf16=dtype == torch.bfloat16)
+    assert (res.mean32.cpu().numpy() == mean32).all()
+    assert (res.centroids.float().cpu().numpy() == cent).all()
+    assert (res.sizes.cpu().numpy() == counts).all()
+    assert torch.equal(norms, centroid_sq(res.centroids))
+    shift = float(np.linalg.norm(cent - old, axis=-1).max())
+    assert abs(float(res.shift.item()) - shift) <= 1e-5 * max(shift, 1.0)
+
+
 def test_centroid_update_accumulates_into_buffers(dev, oracle):
     from sparsepr_amd.flash_kmeans import triton_centroid_update_sorted_euclid
 

@@ -149,3 +149,32 @@ def test_inverse_permutation_of_an_expanded_tensor(dev):
     with pytest.raises(RuntimeError, match="head stride"):
         _lib.call("spr_inverse_permute_rows_strided", _lib.ptr(block), 0, _lib.ptr(idx), _lib.ptr(out), B * H, S,
                   D * 2, _lib.stream(dev))
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 4095, 4096, 4097, 16383, 16384, 16385, 20481])
+@pytest.mark.parametrize("k", [1, 200, 1022, 1023, 1024])
+def test_label_sort_at_its_dispatch_edges(dev, n, k):
+    """One workgroup per row up to 16,384 labels and 1,023 clusters, chunks of 4,096 above;
+    labels outside [0, k) sort last."""
+    from sparsepr_amd.kernels.permute import argsort_labels
+
+    rng = np.random.default_rng(n + k)
+    lab = rng.integers(-1, k + 1, (2, n)).astype(np.int32)
+    lab[1] = rng.integers(0, k, n) // 3 if k > 2 else lab[1]
+    idx, sizes, offsets = (t.cpu().numpy() for t in argsort_labels(torch.from_numpy(lab).to(dev), k))
+    key = np.where((lab >= 0) & (lab < k), lab, k)
+    ref = np.argsort(key, axis=1, kind="stable")
+    want = np.stack([np.bincount(r, minlength=k + 1) for r in key])
+    assert (idx == ref).all() and (sizes == want[:, :k]).all()
+    assert (offsets == np.concatenate((np.zeros((2, 1), int), want[:, :k].cumsum(1)), 1)).all()
+
+
+@pytest.mark.parametrize("k", [2047, 2048, 4095, 4096, 8191])
+def test_label_sort_with_fewer_waves(dev, k):
+    """The scatter's waves per chunk fall from 16 to 2 as their counters grow."""
+    from sparsepr_amd.kernels.permute import argsort_labels
+
+    lab = np.random.default_rng(k).integers(0, k, (3, 9001)).astype(np.int32)
+    idx, sizes, _ = argsort_labels(torch.from_numpy(lab).to(dev), k)
+    assert (idx.cpu().numpy() == np.argsort(lab, axis=1, kind="stable")).all()
+    assert (sizes.cpu().numpy() == np.stack([np.bincount(r, minlength=k) for r in lab])).all()
