@@ -106,6 +106,18 @@ int spr_centroid_mean(const void* x, int32_t dtype, const int32_t* sorted_idx, c
                       const void* old, int64_t batch, int64_t n, int32_t k, int32_t d, float* mean32, void* out,
                       float* shift_max, float* sums_accum, int32_t* counts_accum, float* c_sq_out,
                       void* workspace, size_t workspace_bytes, hipStream_t stream);
+/* The Lloyd loop of kmeans_triton_impl.py:84-115: `iters` times assign, stable label sort and
+ * centroid mean, from init [batch,k,d] (dtype 0 bf16 / 2 fp32, as x).  c_sq fp32 [batch,k]
+ * (nullable: computed) are init's squared norms; x_sq, x_sq_mode and x_sq_out as for
+ * spr_kmeans_assign_bf16 (without x_sq the first iteration's norms serve the later ones).
+ * Outputs: labels, sorted_idx, sizes and offsets of the last assignment, cent [batch,k,d] (not
+ * init's buffer) of the last update, and, nullable, its c_sq_out, mean32 and shift_max as
+ * spr_centroid_mean writes them. */
+size_t spr_lloyd_workspace(int64_t batch, int64_t n, int32_t k, int32_t d, int32_t dtype, int32_t iters);
+int spr_lloyd(const void* x, int32_t dtype, const void* init, const float* c_sq, const float* x_sq, int32_t x_sq_mode,
+              float* x_sq_out, int64_t batch, int64_t n, int32_t k, int32_t d, int32_t iters, int32_t* labels,
+              int32_t* sorted_idx, int32_t* sizes, int32_t* offsets, void* cent, float* c_sq_out, float* mean32,
+              float* shift_max, void* workspace, size_t workspace_bytes, hipStream_t stream);
 /* operator_kmeans.py:609-679 original_centroids / joint_original_centroids, centroid_reduction.py:
  * 138-196 original_centroids_triton / joint_original_centroids_triton: fp32 means of the rows of
  * x (and of y, nullable, in the same traversal of the sorted index) per cluster, fp64 sums;

@@ -42,6 +42,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "spr_centroid_mean_workspace": (_sz, [_i64, _i64, _i32, _i32]),
     "spr_centroid_mean": (ctypes.c_int, [_vp, _i32, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp,
                                          _vp, _vp, _sz, _vp]),
+    "spr_lloyd_workspace": (_sz, [_i64, _i64, _i32, _i32, _i32, _i32]),
+    "spr_lloyd": (ctypes.c_int, [_vp, _i32, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp,
+                                 _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "spr_original_centroids_workspace": (_sz, [_i64, _i64, _i32, _i32]),
     "spr_original_centroids": (ctypes.c_int, [_vp, _vp, _i32, _vp, _vp, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp,
                                               _vp, _sz, _vp]),

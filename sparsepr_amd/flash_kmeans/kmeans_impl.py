@@ -1,6 +1,7 @@
 """Batched Euclidean Lloyd iterations on the HIP kernels of csrc/spr_kmeans.hip.
 
-One iteration is four launches and no host synchronisation (unless tol > 0):
+One iteration is four steps and no host synchronisation (unless tol > 0), all of a loop's
+enqueued by one call (spr_lloyd):
   1. c_sq = ||c||^2 (fp32)                       spr_centroid_sq
   2. labels = argmin distance (bf16 MFMA)         spr_kmeans_assign_bf16
      or, for fp32 inputs, with the TF32 dot      spr_kmeans_assign_tf32
@@ -174,30 +175,42 @@ def lloyd(x: torch.Tensor, n_clusters: int, max_iters: int, tol: float = 0.0,
         cent = random_init(x, K)
     else:
         cent = init_centroids.reshape(B, K, D).to(x.dtype).contiguous()
-    from ..kernels.permute import argsort_labels
-
+    if x.dtype not in _lib.DTYPE_CODE or x.dtype == torch.float16:
+        raise RuntimeError(f"lloyd: unsupported dtype {x.dtype} (bfloat16 or float32)")
     labels = torch.empty((B, N), dtype=torch.int32, device=dev)
-    # squared point norms: computed by the first assignment, reused afterwards
-    cached_sq = None
-    if x_sq is None and max_iters > 1:
-        cached_sq = torch.empty((B, N), dtype=torch.float32, device=dev)
-    res = None
-    it = -1
-    # centroid norms: computed once, then produced by each update for the next assignment
-    c_sq = centroid_sq(cent)
+    sorted_idx = torch.empty((B, N), dtype=torch.int32, device=dev)
+    sizes = torch.empty((B, K), dtype=torch.int32, device=dev)
+    offsets = torch.empty((B, K + 1), dtype=torch.int32, device=dev)
+    mean32 = torch.empty((B, K, D), dtype=torch.float32, device=dev) if want_mean32 else None
+    xs = None if x_sq is None else x_sq.to(torch.float32).contiguous()
+    code = _lib.DTYPE_CODE[x.dtype]
+
+    def run(iters, init, c_sq, norms, norms_out, c_sq_out, shift):
+        """`iters` iterations from `init` in one call; returns the last centroids."""
+        out = torch.empty_like(init)
+        ws = _lib.workspace(_lib.query("spr_lloyd_workspace", B, N, K, D, code, iters), dev)
+        _lib.call("spr_lloyd", _lib.ptr(x), code, _lib.ptr(init), _lib.ptr(c_sq), _lib.ptr(norms), int(x_sq_mode),
+                  _lib.ptr(norms_out), B, N, K, D, iters, _lib.ptr(labels), _lib.ptr(sorted_idx), _lib.ptr(sizes),
+                  _lib.ptr(offsets), _lib.ptr(out), _lib.ptr(c_sq_out), _lib.ptr(mean32), _lib.ptr(shift),
+                  _lib.ptr(ws), ws.numel(), _lib.stream(dev))
+        return out
+
+    if tol <= 0 and not verbose:
+        cent = run(max_iters, cent, None, xs, None, None, None)
+        return LloydResult(labels, cent, sizes, max_iters, sorted_idx, offsets, mean32)
+    # the stop test reads the centroid movement after every iteration: one call for each; the
+    # point norms of the first serve the later ones, as do the centroid norms of each update
+    kept = torch.empty((B, N), dtype=torch.float32, device=dev) if xs is None and max_iters > 1 else None
+    c_sq = None
     for it in range(max_iters):
-        if x_sq is None and cached_sq is not None and it > 0:
-            euclid_assign(x, cent, cached_sq, x_sq_mode=x_sq_mode, c_sq=c_sq, out=labels)
-        else:
-            euclid_assign(x, cent, x_sq, x_sq_mode=x_sq_mode, c_sq=c_sq, out=labels, x_sq_out=cached_sq)
-        sorted_idx, sizes, offsets = argsort_labels(labels, K)
-        next_sq = torch.empty((B, K), dtype=torch.float32, device=dev) if c_sq is not None else None
-        res = centroid_update_sorted(x, labels, cent, want_mean32=want_mean32, want_shift=tol > 0 or verbose,
-                                     sorted_idx=sorted_idx, sizes=sizes, offsets=offsets, c_sq_out=next_sq)
-        c_sq = next_sq
+        norms = xs if xs is not None else (kept if it > 0 else None)
+        c_sq_out = torch.empty((B, K), dtype=torch.float32, device=dev)
+        shift = torch.zeros(1, dtype=torch.float32, device=dev)
+        new = run(1, cent, c_sq, norms, kept if norms is None else None, c_sq_out, shift)
+        moved = float(shift.item())
         if verbose:
-            print(f"Iter {it}, center shift: {float(res.shift.item()):.6f}")
-        if tol > 0 and float(res.shift.item()) < tol:
-            return LloydResult(labels, cent, sizes, it + 1, sorted_idx, offsets, res.mean32)
-        cent = res.centroids
-    return LloydResult(labels, cent, res.sizes, it + 1, res.sorted_idx, res.offsets, res.mean32)
+            print(f"Iter {it}, center shift: {moved:.6f}")
+        if tol > 0 and moved < tol:
+            return LloydResult(labels, cent, sizes, it + 1, sorted_idx, offsets, mean32)
+        cent, c_sq = new, c_sq_out
+    return LloydResult(labels, cent, sizes, max_iters, sorted_idx, offsets, mean32)

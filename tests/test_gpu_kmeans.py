@@ -141,6 +141,31 @@ def test_centroid_mean_of_short_inputs(dev, oracle, n, dtype, d):
     assert abs(float(res.shift.item()) - shift) <= 1e-5 * max(shift, 1.0)
 
 
+@pytest.mark.parametrize("iters", [1, 2, 3])  # the centroids alternate between two buffers
+@pytest.mark.parametrize("dtype,d,n", [(torch.bfloat16, 64, 500), (torch.bfloat16, 128, 9000), (torch.float32, 48, 9000)])
+def test_lloyd_in_one_call_equals_its_steps(dev, oracle, iters, dtype, d, n):
+    """The whole loop against assign, sort and mean called one by one: the same bits."""
+    from sparsepr_amd.flash_kmeans.kmeans_impl import centroid_sq, centroid_update_sorted, euclid_assign, lloyd
+    from sparsepr_amd.kernels.permute import argsort_labels
+
+    rng = np.random.default_rng(n + iters)
+    x = to_dev(_gmm(oracle, rng, 2, n, d, 12), dev, dtype)
+    init = x[:, :17].contiguous()
+    res = lloyd(x, 17, iters, 0.0, init, want_mean32=True)
+    stop = lloyd(x, 17, iters, 1e-30, init, want_mean32=True)  # a call per iteration
+    cent, norms = init, torch.empty((2, n), device=dev)
+    for it in range(iters):
+        labels = euclid_assign(x, cent, norms if it else None, c_sq=centroid_sq(cent), x_sq_out=None if it else norms)
+        idx, sizes, off = argsort_labels(labels, 17)
+        up = centroid_update_sorted(x, labels, cent, want_mean32=True, sorted_idx=idx, sizes=sizes, offsets=off)
+        cent = up.centroids
+    for got in (res, stop) if stop.iters == iters and not torch.equal(stop.centroids, init) else (res,):
+        assert torch.equal(got.labels, labels) and torch.equal(got.sorted_idx, idx)
+        assert torch.equal(got.sizes, sizes) and torch.equal(got.offsets, off)
+        assert torch.equal(got.centroids, cent) and torch.equal(got.mean32, up.mean32)
+    assert torch.equal(init, x[:, :17])
+
+
 def test_centroid_update_accumulates_into_buffers(dev, oracle):
     from sparsepr_amd.flash_kmeans import triton_centroid_update_sorted_euclid
 
