@@ -318,7 +318,7 @@ def only_role_proj(args):
     ms = start.elapsed_time(end) / args.steps
     nbytes = x.numel() * 2 + out.numel() * 4 + factor.numel() * 4
     gbs = nbytes / ms / 1e6
-    print(json.dumps({"kernel": "role_projection_kernel<128, 2>", "ms_per_launch": round(ms, 4),
+    print(json.dumps({"kernel": "role_projection_rows_kernel<128, 64>", "ms_per_launch": round(ms, 4),
                       "config": {"bh": B * H, "tokens": N, "head_dim": D, "rank": 64},
                       "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                    "frac": round(gbs / HBM_PEAK_GBS, 4), "bytes_per_launch": nbytes}}), flush=True)

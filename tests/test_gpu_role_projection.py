@@ -157,3 +157,37 @@ def test_role_kv_projection_and_init(dev, oracle, precision):
     ref_init = np.concatenate((oracle.project_rows(kc, kf, rks.reshape(-1), precision=precision),
                                oracle.project_rows(vc, vf, rvs.reshape(-1), precision=precision, weight=w)), axis=2)
     assert np.abs(init.cpu().numpy() - ref_init).max() <= 1e-4 * np.abs(ref_init).max()
+
+
+@pytest.mark.parametrize("bh,n,d,r,precision", [
+    (32, 8192, 128, 64, "highest"), (32, 8193, 64, 16, "medium"), (31, 8479, 128, 48, "highest"),
+    (32, 8223, 64, 32, "high"), (1, 262145, 128, 16, "medium"), (260, 8225, 64, 48, "high"),
+    (31, 8192, 128, 64, "high")])
+def test_long_projections_at_tile_and_unit_edges(dev, oracle, bh, n, d, r, precision):
+    """Long calls at whole and ragged 32-token tiles and 256-token units, shares that cross heads,
+    more heads than CUs, and one call just too short for the streaming kernel: the rows of three
+    heads at both ends and around the units' edges, with the features beside other columns."""
+    from sparsepr_amd.kernels.role_projection import role_k_projection_normalize, role_projection_rms_triton
+
+    g = torch.Generator(device=dev).manual_seed(n + r)
+    x = torch.randn((bh, n, d), device=dev, generator=g).to(torch.bfloat16)
+    x[bh // 2, n - 1] = 0.0
+    f = torch.randn((bh, d, r), device=dev, generator=g) / d ** 0.5
+    print(f"long projection bh={bh} n={n} d={d} r={r}", flush=True)
+    rms = role_projection_rms_triton(x, f)
+    wide = torch.full((bh, n, r + 8), 7.0, device=dev)
+    _, scale = role_k_projection_normalize(x, f, precision=precision, weight=0.35, out=wide, out_col=4)
+    feat = wide[:, :, 4:4 + r]
+    again, _ = role_k_projection_normalize(x, f, precision=precision, weight=0.35)
+    torch.cuda.synchronize()
+    assert torch.equal(feat, again)
+    assert (wide[:, :, :4] == 7.0).all() and (wide[:, :, 4 + r:] == 7.0).all()
+    rows = sorted({*range(0, 70), *range(n // 2 // 256 * 256 - 35, n // 2 // 256 * 256 + 35), *range(n - 70, n)})
+    for h in sorted({0, bh // 2, bh - 1}):
+        xs = x[h:h + 1].float().cpu().numpy()
+        fs = f[h:h + 1].cpu().numpy()
+        ref_rms = oracle.role_projection_rms(xs[:, rows], fs)
+        assert np.abs(rms[h:h + 1, rows].cpu().numpy().astype(np.float64) - ref_rms).max() < ATOL
+        ref, ref_scale = oracle.role_k_projection_normalize(xs, fs, precision, 0.35)
+        assert abs(scale[h].item() - float(np.ravel(ref_scale)[0])) < 1e-5 * float(np.ravel(ref_scale)[0])
+        assert np.abs(feat[h].cpu().numpy().astype(np.float64) - ref[0]).max() < ATOL
