@@ -67,6 +67,14 @@ __device__ __forceinline__ float tf32_rna(float x) {
 
 __device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * SE_LOG2E); }
 
+// log(x) + y for x >= 0, rounded once: with the reference at the centroid logit the two can be large
+// and of opposite signs, and a log rounded by itself would show in a small score.
+__device__ __forceinline__ float log_plus(float x, double y) {
+  int e = 0;
+  const float m = frexpf(x, &e);
+  return static_cast<float>(y + (0.6931471805599453 * e + static_cast<double>(logf(m))));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
@@ -561,8 +569,9 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
     float score = -__builtin_huge_valf();
     if ((filled >> j) & 1u) {
       // value error: log(max(E / n, 1e-30)) of the weights taken from the largest logit
-      score = MODE == 0 ? fmaxf(logf(total / static_cast<float>(len_l[j])) + 2.0f * ref, -69.07755278982137f + 2.0f * top)
-                        : logf(fmaxf(total, 1.0e-30f)) + ref;
+      score = MODE == 0 ? fmaxf(log_plus(total / static_cast<float>(len_l[j]), 2.0 * ref),
+                                -69.07755278982137f + 2.0f * top)
+                        : log_plus(fmaxf(total, 1.0e-30f), ref);
     }
     scores[(qh * qn + q0 + r) * kn + c_begin + j] = score;
   }
