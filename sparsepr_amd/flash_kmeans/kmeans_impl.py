@@ -174,6 +174,7 @@ def lloyd(x: torch.Tensor, n_clusters: int, max_iters: int, tol: float = 0.0,
     if init_centroids is None:
         cent = random_init(x, K)
     else:
+        _lib.require_gpu(init_centroids, x, what="lloyd: init_centroids")
         cent = init_centroids.reshape(B, K, D).to(x.dtype).contiguous()
     if x.dtype not in _lib.DTYPE_CODE or x.dtype == torch.float16:
         raise RuntimeError(f"lloyd: unsupported dtype {x.dtype} (bfloat16 or float32)")

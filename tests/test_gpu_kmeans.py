@@ -424,3 +424,13 @@ def test_role_step64_exact(dev, oracle):
     assert (labels.cpu().numpy() == rl).all()
     with pytest.raises(RuntimeError):
         role_cluster_step_q64(to_dev(f, dev), to_dev(c2, dev))  # 1000 > 512 clusters
+
+
+@pytest.mark.parametrize("tol", [0.0, 1e-3])
+def test_lloyd_refuses_host_centroids(dev, tol):
+    """The loop hands its pointers to the kernels: centroids in host memory are refused before it."""
+    from sparsepr_amd.flash_kmeans.kmeans_impl import lloyd
+
+    x = torch.zeros((1, 64, 64), dtype=torch.bfloat16, device=dev)
+    with pytest.raises(RuntimeError, match="require GPU tensors"):
+        lloyd(x, 4, 2, tol, torch.zeros((1, 4, 64), dtype=torch.bfloat16))
