@@ -1066,8 +1066,8 @@ __global__ __launch_bounds__(256) void mean_slice_plan_kernel(const int32_t* __r
 }
 
 // T: uint16_t (bf16) or float.  Workgroup (s, b) sums slice s of batch b (rows
-// slice_rows[b][s] of the sorted order; without a plan, cluster s) in fp64.  The one slice of a cluster finalizes its
-// mean directly; otherwise the sum goes to partial[b][s][D], and
+// slice_rows[b][s] of the sorted order; without a plan, cluster s) in fp64.  The one slice of
+// a cluster finalizes its mean directly; otherwise the sum goes to partial[b][s][D], and
 // centroid_mean_finalize_kernel adds the cluster's slices in order (the result does not
 // depend on the split).
 template <typename T, int D>

@@ -239,8 +239,9 @@ __global__ __launch_bounds__(RP_THREADS) void role_projection_kernel(const uint1
 // likewise.  Factor fragments are read four ahead of their MFMA: left to itself the compiler
 // read each right before its use, some 130 cycles apart.
 // 24 heads x 118,800 tokens, D = 128: rank 64 with row RMS 330 -> 304 us, rank 48 with the head's
-// RMS 205 + 320 -> 186 + 262 us (the first 4.4 -> 4.8 TB/s); a call of both 793 -> 731 us.  Twelve waves 808 us, four with a triple DMA buffer 766, eight with two
-// tiles ahead 746, the factor in registers 963 (it spills).
+// RMS 205 + 320 -> 186 + 262 us (the first 4.4 -> 4.8 TB/s); a call of both 793 -> 731 us.
+// Twelve waves 808 us, four with a triple DMA buffer 766, eight with two tiles ahead 746, the
+// factor in registers 963 (it spills).
 constexpr int RS_WAVES = 8;
 // tokens of a unit: one tile, or 256 in the sum pass, which leaves one fp64 partial for each
 constexpr int rs_unit(int mode) { return mode == 1 ? 256 : 32; }
