@@ -602,7 +602,7 @@ def bench_layer(args, name, top_p=None, repair=True, amp=None, with_cpu=False):
         "stages_ms": stage_ms,
         "roofline": {
             "kernel": "attn_pipe_kernel (D=128 block-sparse attention)" if d == 128
-            else "attn_pipe_kernel<64> (D=64 block-sparse attention)",
+            else "attn_fwd_kernel<64> (D=64 block-sparse attention)",
             "bound": "mfma",
             "achieved": round(achieved, 1),
             "peak": MFMA_BF16_PEAK_TFLOPS,

@@ -28,9 +28,9 @@
 // (key(t, h, e) = 16t + 8(e/4) + 4h + e%4), which makes P a plain slice of the
 // accumulator.
 //
-// Kernels: attn_pipe_kernel (D = 128 and 64 block-sparse: 256-row tiles, K/V DMA'd
+// Kernels: attn_pipe_kernel (D = 128 block-sparse: 256-row tiles, K/V DMA'd
 // into swizzled LDS tiles, next-S/softmax pipelining) and attn_fwd_kernel
-// (D = 16 and 32 block-sparse and the dense probe attention: 128-row tiles, K/V
+// (D = 16, 32 and 64 block-sparse and the dense probe attention: 128-row tiles, K/V
 // staged through registers into a padded K tile and a transposed V tile,
 // double-buffered, the next chunk fetched while the current one computes).
 #include "spr_common.h"
@@ -746,7 +746,7 @@ __global__ __launch_bounds__(NW * 64, QB == 2 ? 1 : 2) void attn_fwd_kernel(
   }
 }
 
-// ---------------------------------------------------------------------------- block-sparse, D = 128 and 64: LDS layout
+// ---------------------------------------------------------------------------- block-sparse, D = 128: LDS layout
 // K and V chunks are copied from HBM straight into LDS (buffer_load ... lds, 16
 // bytes a lane, 1 KB per wave instruction): no staging registers and no staging
 // work in the waves' instruction streams.
@@ -765,20 +765,12 @@ __global__ __launch_bounds__(NW * 64, QB == 2 ? 1 : 2) void attn_fwd_kernel(
 // accumulator produces (key(t, h, e) = 16t + 8(e/4) + 4h + e%4).  The 4 rows x
 // 4 pieces each half-wave reads (pieces 4b .. 4b + 3) land in 16 distinct
 // slots, all 64 banks.
-//
-// D = 64: rows of 128 bytes, two of which span the banks, so the row pair is what the
-// swizzle uses: piece j of row r at slot j ^ ((r >> 1) & 7) in K and j ^ 4((r >> 1) & 1) in V
-// (rows r and r + 1 already lie 32 banks apart).
-template <int D>
-struct PipeTile {
-  static_assert(D == 64 || D == 128, "swizzles for 128- and 256-byte rows");
-  static constexpr int ROW = 2 * D;           // bytes per key row
-  static constexpr int BYTES = BN * ROW;      // bytes per K or V chunk tile
-  static constexpr int PIECES = ROW / 16;     // 16-byte pieces per row
-  static constexpr int DMA_ROWS = 64 / PIECES;  // rows one wave's DMA instruction moves
-  __device__ static __forceinline__ int k_swz(int r) { return D == 128 ? r & 15 : (r >> 1) & 7; }
-  __device__ static __forceinline__ int v_swz(int r) { return D == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2; }
-};
+constexpr int DROW = 256;             // bytes per key row (D = 128)
+constexpr int DTILE = BN * DROW;      // bytes per K or V chunk tile
+constexpr int DPIECES = DROW / 16;    // 16-byte pieces per row
+constexpr int DMA_ROWS = 64 / DPIECES;  // rows one wave's DMA instruction moves
+__device__ __forceinline__ int k_swz(int r) { return r & 15; }
+__device__ __forceinline__ int v_swz(int r) { return (r & 3) << 2; }
 
 struct alignas(8) u32x2 {
   uint32_t x, y;
@@ -794,7 +786,7 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint8_t* p) {
 #endif
 }
 
-// ---------------------------------------------------------------------------- block-sparse, D = 128 and 64, pipelined
+// ---------------------------------------------------------------------------- block-sparse, D = 128, pipelined
 // The work items, plan walk and online softmax of attn_fwd_kernel MODE 0 over
 // 256-row query tiles: eight waves of 32 rows (two per SIMD, one workgroup per
 // CU) share each K/V chunk, which halves the HBM/L2 traffic and DMA issue per
@@ -814,27 +806,18 @@ __host__ __device__ inline int32_t tile_turns(int64_t tiles) {
   return static_cast<int32_t>((tiles + 8 * TILE_RUN - 1) / (8 * TILE_RUN));
 }
 
-template <int D, bool KIDX, bool F16>
-__global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
+template <bool KIDX, bool F16>
+__global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int32_t s_q,
     int32_t s_kv, int32_t group, int32_t qn, int32_t kn, const int32_t* __restrict__ plan, int32_t bh_q,
     int32_t tiles_per_head, float scale_log2, const int32_t* __restrict__ q_index,
     const int32_t* __restrict__ k_index, uint16_t* __restrict__ out, float* __restrict__ lse) {
   constexpr int NW = 8;
-  // D = 128: S of the next half is computed beside the softmax of the current one, two waves
-  // per SIMD.  D = 64: half the MFMAs meet the same softmax, which is then the bound; the plain
-  // S, softmax, P V order leaves registers for four waves per SIMD (two workgroups per CU)
-  // that cover one another (12 heads x 40,000 tokens, density 0.2: 1.26 to 1.39 ms, box to box,
-  // as the register-staged kernel took; computed ahead it is 15 % slower at two waves and
-  // 31 % at four, with spills).
-  constexpr bool AHEAD = D == 128;
-  using T = PipeTile<D>;
-  constexpr int DROW = T::ROW;
-  constexpr int DTILE = T::BYTES;
+  constexpr int D = 128;
   constexpr int KSTEPS = D / 16;
   constexpr int DBLK = D / 32;
   constexpr int TBM = NW * 32;
-  constexpr int DMA_PER_WAVE = BN / T::DMA_ROWS / NW;
+  constexpr int DMA_PER_WAVE = BN / DMA_ROWS / NW;
   __shared__ __attribute__((aligned(1024))) uint8_t k_tiles[4][DTILE];
   uint8_t* const k_tile0 = k_tiles[0];
   uint8_t* const k_tile1 = k_tiles[1];
@@ -947,7 +930,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
     int32_t vpos[DMA_PER_WAVE];
 #pragma unroll
     for (int i = 0; i < DMA_PER_WAVE; ++i) {
-      vpos[i] = min(c * BN + T::DMA_ROWS * (wave + NW * i) + lane / T::PIECES, total - 1);
+      vpos[i] = min(c * BN + DMA_ROWS * (wave + NW * i) + lane / DPIECES, total - 1);
       krow[i] = cur_delta;
     }
     // the list's last end is `total`, so the walk stays inside it
@@ -969,22 +952,22 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
     }
   };
   auto dma = [&](uint8_t* kt, uint8_t* vt) {
-    const int slot = lane % T::PIECES;
+    const int slot = lane % DPIECES;
 #pragma unroll
     for (int i = 0; i < DMA_PER_WAVE; ++i) {
-      const int r0 = T::DMA_ROWS * (wave + NW * i);
-      const int row = r0 + lane / T::PIECES;
+      const int r0 = DMA_ROWS * (wave + NW * i);
+      const int row = r0 + lane / DPIECES;
       const int32_t off = krow[i] * DROW;
-      spr::lds_dma16(k_desc, kt + r0 * DROW, off + ((slot ^ T::k_swz(row)) << 4));
-      spr::lds_dma16(v_desc, vt + r0 * DROW, off + ((slot ^ T::v_swz(row)) << 4));
+      spr::lds_dma16(k_desc, kt + r0 * DROW, off + ((slot ^ k_swz(row)) << 4));
+      spr::lds_dma16(v_desc, vt + r0 * DROW, off + ((slot ^ v_swz(row)) << 4));
     }
   };
 
-  const int k_x = half ^ T::k_swz(col);
+  const int k_x = half ^ k_swz(col);
   const int tr_a = lane & 3, tr_i = (lane >> 2) & 3, tr_g = (lane >> 4) & 1;
   const int v_lane = (4 * half + tr_i) * DROW + (tr_a & 1) * 8;
   const int v_piece = 2 * tr_g + (tr_a >> 1);
-  const int v_x = T::v_swz(tr_i);
+  const int v_x = v_swz(tr_i);
 
   auto s_mma = [&](spr::f32x16& acc, const uint8_t* kt, int kbk) {
     acc = spr::f32x16{};
@@ -1047,17 +1030,15 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
     for (int st = 0; st < KSTEPS; ++st) {
       if (st + 2 < KSTEPS) ka[(st + 2) % 3] = kfrag(st + 2);
       acc_next = mfma16<F16>(ka[st % 3], qf[st], acc_next);
-#pragma unroll
-      for (int e = 16 / KSTEPS * st; e < 16 / KSTEPS * (st + 1); e += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[e], scale_log2, neg_m));
-        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[e + 1], scale_log2, neg_m));
-        const uint32_t pk = pack2t<F16>(p0, p1);
-        pf[e / 8][(e % 8) / 2] = pk;
-        if (e % 4 == 0) {
-          lsum0 = dot2_ones<F16>(pk, lsum0);
-        } else {
-          lsum1 = dot2_ones<F16>(pk, lsum1);
-        }
+      const int e = 2 * st;
+      const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[e], scale_log2, neg_m));
+      const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[e + 1], scale_log2, neg_m));
+      const uint32_t pk = pack2t<F16>(p0, p1);
+      pf[e / 8][(e % 8) / 2] = pk;
+      if (e % 4 == 0) {
+        lsum0 = dot2_ones<F16>(pk, lsum0);
+      } else {
+        lsum1 = dot2_ones<F16>(pk, lsum1);
       }
     }
     l_run += lsum0 + lsum1;
@@ -1174,51 +1155,31 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 1) void attn_pipe_kernel(
       load_rows(2);
       dma(k_tile2, v_tile2);
     }
-    if constexpr (AHEAD) {
-      spr::wait_vm<0>();
-      spr::lds_barrier();  // chunks 0 .. 2 landed
-      if (wave_live) s_mma(s_a, k_tile0, only);
-      if (split) {
-        // One half per chunk: S of this wave's half of chunk x is in s_a; S of the same half
-        // of chunk x + 1 (the next K tile, so after the barrier) goes to s_b.  The barriers,
-        // DMAs and planning are those of the full path.
-        for (int x = 0; x < nch; ++x) {
-          const int32_t left = total - x * BN;
-          if (x + 3 < nch) load_rows(x + 3);
-          if (wave_live) row_max(s_a, only, left);
-          if (x + 2 < nch) spr::wait_vm<2 * DMA_PER_WAVE>(); else spr::wait_vm<0>();
-          spr::lds_barrier();
-          if (wave_live) {
-            step(s_b, k_tiles[(x + 1) & 3], only, s_a, v_tiles[x & 3], only);
-            s_a = s_b;
-          }
-          if (x + 3 < nch) dma(k_tiles[(x + 3) & 3], v_tiles[(x + 3) & 3]);
+    spr::wait_vm<0>();
+    spr::lds_barrier();  // chunks 0 .. 2 landed
+    if (wave_live) s_mma(s_a, k_tile0, only);
+    if (split) {
+      // One half per chunk: S of this wave's half of chunk x is in s_a; S of the same half
+      // of chunk x + 1 (the next K tile, so after the barrier) goes to s_b.  The barriers,
+      // DMAs and planning are those of the full path.
+      for (int x = 0; x < nch; ++x) {
+        const int32_t left = total - x * BN;
+        if (x + 3 < nch) load_rows(x + 3);
+        if (wave_live) row_max(s_a, only, left);
+        if (x + 2 < nch) spr::wait_vm<2 * DMA_PER_WAVE>(); else spr::wait_vm<0>();
+        spr::lds_barrier();
+        if (wave_live) {
+          step(s_b, k_tiles[(x + 1) & 3], only, s_a, v_tiles[x & 3], only);
+          s_a = s_b;
         }
-      } else {
-        for (int x = 0; x < nch; x += 4) {
-          chunk(x, k_tile0, v_tile0, k_tile1, k_tile3, v_tile3);
-          if (x + 1 < nch) chunk(x + 1, k_tile1, v_tile1, k_tile2, k_tile0, v_tile0);
-          if (x + 2 < nch) chunk(x + 2, k_tile2, v_tile2, k_tile3, k_tile1, v_tile1);
-          if (x + 3 < nch) chunk(x + 3, k_tile3, v_tile3, k_tile0, k_tile2, v_tile2);
-        }
+        if (x + 3 < nch) dma(k_tiles[(x + 3) & 3], v_tiles[(x + 3) & 3]);
       }
     } else {
-      for (int x = 0; x < nch; ++x) {
-        // this wave's DMA of chunk x landed; those of chunks x + 1 and x + 2 may be in flight
-        if (x + 2 < nch) spr::wait_vm<4 * DMA_PER_WAVE>(); else if (x + 1 < nch) spr::wait_vm<2 * DMA_PER_WAVE>(); else spr::wait_vm<0>();
-        spr::lds_barrier();  // ... every wave's; and no wave reads chunk x - 1, whose tiles are next
-        if (x + 3 < nch) {
-          load_rows(x + 3);
-          dma(k_tiles[(x + 3) & 3], v_tiles[(x + 3) & 3]);
-        }
-        if (wave_live) {
-          const int32_t left = total - x * BN;
-          for (int h = only; h < (split ? only + 1 : 2); ++h) {
-            s_mma(s_a, k_tiles[x & 3], h);
-            row_max(s_a, h, left);
-            pv_step(s_a, v_tiles[x & 3], h);
-          }
-        }
+      for (int x = 0; x < nch; x += 4) {
+        chunk(x, k_tile0, v_tile0, k_tile1, k_tile3, v_tile3);
+        if (x + 1 < nch) chunk(x + 1, k_tile1, v_tile1, k_tile2, k_tile0, v_tile0);
+        if (x + 2 < nch) chunk(x + 2, k_tile2, v_tile2, k_tile3, k_tile1, v_tile1);
+        if (x + 3 < nch) chunk(x + 3, k_tile3, v_tile3, k_tile0, k_tile2, v_tile2);
       }
     }
   }
@@ -1561,24 +1522,20 @@ extern "C" int spr_block_sparse_attention_run_ex(const void* q, const void* k, c
   const int32_t* pl = static_cast<const int32_t*>(plan);
   uint16_t* o16 = static_cast<uint16_t*>(out);
   const int32_t s32 = static_cast<int32_t>(s), bhq32 = static_cast<int32_t>(bh_q);
-  if (d == 128 || d == 64) {
+  if (d == 128) {
     const int64_t max_tiles_pipe = spr::ceil_div(s, 2 * BM) + qn;
     const int64_t pipe_blocks = static_cast<int64_t>(tile_turns(max_tiles_pipe)) * TILE_RUN * 8 * bh_q;
     SPR_REQUIRE(pipe_blocks < (int64_t(1) << 31), "spr_block_sparse_attention_run: too many tiles");
     dim3 grid_pipe(static_cast<uint32_t>(pipe_blocks));
     const int32_t tph = static_cast<int32_t>(max_tiles_pipe);
-    auto pipe = [&](auto dd, auto kxc, auto f) {
-      attn_pipe_kernel<decltype(dd)::value, decltype(kxc)::value, decltype(f)::value><<<grid_pipe, 512, 0, stream>>>(
+    auto pipe = [&](auto kxc, auto f) {
+      attn_pipe_kernel<decltype(kxc)::value, decltype(f)::value><<<grid_pipe, 512, 0, stream>>>(
           q16, k16, v16, s32, s32, group, qn, kn, pl, bhq32, tph, scale_log2, q_index, k_index, o16, lse);
     };
-    auto pipe_by_flags = [&](auto dd) {
-      using T_ = std::true_type;
-      using F_ = std::false_type;
-      if (kx) { f16 ? pipe(dd, T_{}, T_{}) : pipe(dd, T_{}, F_{}); }
-      else    { f16 ? pipe(dd, F_{}, T_{}) : pipe(dd, F_{}, F_{}); }
-    };
-    if (d == 128) pipe_by_flags(std::integral_constant<int, 128>{});
-    else pipe_by_flags(std::integral_constant<int, 64>{});
+    using T_ = std::true_type;
+    using F_ = std::false_type;
+    if (kx) { f16 ? pipe(T_{}, T_{}) : pipe(T_{}, F_{}); }
+    else    { f16 ? pipe(F_{}, T_{}) : pipe(F_{}, F_{}); }
     SPR_LAUNCHED("attn_pipe_kernel");
     return SPR_OK;
   }
@@ -1599,7 +1556,8 @@ extern "C" int spr_block_sparse_attention_run_ex(const void* q, const void* k, c
       else    { f16 ? fwd(dd, F_{}, F_{}, T_{}) : fwd(dd, F_{}, F_{}, F_{}); }
     }
   };
-  if (d == 32) by_flags(std::integral_constant<int, 32>{});
+  if (d == 64) by_flags(std::integral_constant<int, 64>{});
+  else if (d == 32) by_flags(std::integral_constant<int, 32>{});
   else by_flags(std::integral_constant<int, 16>{});
   SPR_LAUNCHED("attn_fwd_kernel");
   return SPR_OK;

@@ -151,6 +151,23 @@ def test_block_sparse_segment_walk(dev, oracle, D, kn, size):
     assert np.abs(got.float().cpu().numpy() - ref[0]).max() <= ATOL
 
 
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float16), (32, torch.bfloat16)])
+def test_small_head_rows_do_not_depend_on_their_tile(dev, D, dtype):
+    """Up to head dim 64 a wave takes all keys of its rows in order: the same bits whether a row's
+    q-cluster has one 32-row block, two, four or more."""
+    from sparsepr_amd.kernels.attention import block_sparse_attention
+
+    g = torch.Generator(device=dev).manual_seed(D)
+    S = 330
+    q, k, v = (torch.randn((1, S, D), device=dev, generator=g).to(dtype) for _ in range(3))
+    m = torch.ones((1, 2, 3), dtype=torch.bool, device=dev)
+    ks = torch.tensor([[37, 193, 100]], device=dev)
+    outs = [block_sparse_attention(q, k, v, m, torch.tensor([[rows, S - rows]], device=dev), ks, return_lse=True)
+            for rows in (31, 64, 100, 161, 256, 300)]
+    for out, lse in outs[1:]:
+        assert torch.equal(out, outs[0][0]) and torch.equal(lse, outs[0][1])
+
+
 @pytest.mark.parametrize("D,f16,Hq,Hkv", [(16, False, 2, 2), (32, False, 4, 2), (16, True, 2, 2), (32, True, 2, 2),
                                          (64, True, 4, 2), (128, True, 2, 2)])
 def test_block_sparse_head_dims_and_fp16(dev, oracle, D, f16, Hq, Hkv):
