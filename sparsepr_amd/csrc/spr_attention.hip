@@ -958,8 +958,8 @@ __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
       const int r0 = DMA_ROWS * (wave + NW * i);
       const int row = r0 + lane / DPIECES;
       const int32_t off = krow[i] * DROW;
-      spr::lds_dma16(k_desc, kt + r0 * DROW, off + ((slot ^ k_swz(row)) << 4));
-      spr::lds_dma16(v_desc, vt + r0 * DROW, off + ((slot ^ v_swz(row)) << 4));
+      spr::lds_dma16x2(k_desc, kt + r0 * DROW, off + ((slot ^ k_swz(row)) << 4), v_desc, vt + r0 * DROW,
+                       off + ((slot ^ v_swz(row)) << 4));
     }
   };
 

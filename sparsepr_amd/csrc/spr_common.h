@@ -119,16 +119,28 @@ __device__ __forceinline__ i32x4_s buffer_desc(const void* p, int32_t bytes) {
                  __builtin_amdgcn_readfirstlane(bytes), 0x00020000};
 }
 
-// 16 bytes a lane from buffer offset voff to lds + 16 * lane (lds wave-uniform).  Written out
-// because the compiler tracks the builtin's write to LDS: it then waits for every DMA in
+// 16 bytes a lane from buffer offset voff to lds + 16 * lane (lds wave-uniform), twice.  Written
+// out because the compiler tracks the builtin's write to LDS: it then waits for every DMA in
 // flight at each barrier and before most LDS reads of the tiles, which ends the prefetch.
-// Nothing tracks this one: a reader waits by s_waitcnt vmcnt and a barrier.
-__device__ __forceinline__ void lds_dma16(i32x4_s desc, const uint8_t* lds, int32_t voff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const int32_t base = __builtin_amdgcn_readfirstlane(
+// Nothing tracks this one: a reader waits by s_waitcnt vmcnt and a barrier.  The compiler places no
+// waits inside the block either: a buffer instruction may read an SGPR five wait states after a
+// VALU write (a descriptor put together by v_readlane), two moves and s_nop 2 here, and m0 one
+// after its write.  m0 is given back: the compiler may hold a base of its own there.  Two to a
+// block share the wait: one each costs the attention of the 24 x 118,800 layer 1.2 %.
+__device__ __forceinline__ int32_t lds_base(const uint8_t* lds) {
+  return __builtin_amdgcn_readfirstlane(
       static_cast<int32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)lds)));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(base), "v"(voff), "s"(desc) : "memory");
+}
+__device__ __forceinline__ void lds_dma16x2(i32x4_s desc0, const uint8_t* lds0, int32_t voff0, i32x4_s desc1,
+                                            const uint8_t* lds1, int32_t voff1) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  int32_t kept;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 2\n\t"
+               "buffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %4\n\ts_nop 0\n\t"
+               "buffer_load_dwordx4 %5, %6, 0 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(kept)
+               : "s"(lds_base(lds0)), "v"(voff0), "s"(desc0), "s"(lds_base(lds1)), "v"(voff1), "s"(desc1)
+               : "memory");
 #endif
 }
 

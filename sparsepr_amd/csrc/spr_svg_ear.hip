@@ -326,15 +326,13 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
       spr::buffer_desc(MODE == 0 ? vs + kh * t_stored * SE_D : ks, static_cast<int32_t>(t_stored * SE_ROW));
   auto dma = [&](const Walk& w, int kt, int vt) {
     if (wave < 4) {
-      const int slot = lane & 15;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int r0 = 4 * wave + 16 * i;
-        const int row = r0 + (lane >> 4);
-        const int32_t off = (w.start + w.c0 + row) * SE_ROW + ((slot ^ (row & 15)) << 4);
-        spr::lds_dma16(k_desc, k_tiles + kt + r0 * SE_ROW, off);
-        if (MODE == 0) spr::lds_dma16(v_desc, v_tiles + vt + r0 * SE_ROW, off);
-      }
+      const int r0 = 4 * wave, row = r0 + (lane >> 4);  // and 16 rows on, where the swizzle is the same
+      const int32_t off = (w.start + w.c0 + row) * SE_ROW + (((lane ^ row) & 15) << 4);
+      auto rows = [&](spr::i32x4_s desc, const uint8_t* tile) {
+        spr::lds_dma16x2(desc, tile + r0 * SE_ROW, off, desc, tile + (r0 + 16) * SE_ROW, off + 16 * SE_ROW);
+      };
+      rows(k_desc, k_tiles + kt);
+      if (MODE == 0) rows(v_desc, v_tiles + vt);
     }
   };
   constexpr int DMA_PER_CHUNK = MODE == 0 ? 4 : 2;  // per wave that moves any

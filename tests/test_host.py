@@ -1,5 +1,11 @@
-"""Host-side logic of the Python drop-ins that needs no GPU: configuration checks
-and the refusals of configurations that have no HIP path."""
+"""Host-side logic of the Python drop-ins that needs no GPU: configuration checks and
+the refusals of configurations that have no HIP path, and what the compiler makes of the
+inline LDS DMA."""
+
+import re
+import shutil
+import subprocess
+from pathlib import Path
 
 import pytest
 
@@ -30,3 +36,56 @@ def test_route_feature_dims_the_kernels_take():
                      (N8V6Config(), 96)):
         with pytest.raises(NotImplementedError, match="multiple of 16"):
             N8V6Core(cfg, validate=False)._check_route_config(dim)
+
+
+# A descriptor put together by v_readlane right before the inline DMA, and the compiler's own DMA,
+# with the same LDS base before and after it.
+_DMA_PROBE = """
+#include "spr_common.h"
+__global__ void probe(const int32_t* words, const int32_t* src, int32_t* out, int lane) {
+  __shared__ __attribute__((aligned(1024))) int32_t tile[640];
+  const int32_t w = words[threadIdx.x], voff = 16 * threadIdx.x;
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(src), 0, 4096, 0x00020000);
+  auto tracked = [&] {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)tile, 16, voff, 0, 0, 0);
+  };
+  tracked();
+  const spr::i32x4_s desc = {__builtin_amdgcn_readlane(w, lane), __builtin_amdgcn_readlane(w, lane + 1),
+                             __builtin_amdgcn_readlane(w, lane + 2), 0x00020000};
+  const uint8_t* half = reinterpret_cast<uint8_t*>(tile + 256);
+  spr::lds_dma16x2(desc, half, voff, desc, half + 512, voff + 512);
+  tracked();
+  spr::wait_vm<0>();
+  spr::lds_barrier();
+  out[threadIdx.x] = tile[threadIdx.x] + tile[256 + threadIdx.x];
+}
+"""
+
+
+def test_inline_dma_states_what_it_reads_and_writes(tmp_path):
+    """The DMA's asm block waits for a descriptor that a VALU instruction has just written (five
+    wait states) and leaves m0 to the compiler, whose own DMA behind it relies on the base that it
+    set before."""
+    from sparsepr_amd import build_hip
+
+    if shutil.which(build_hip.HIPCC) is None:
+        pytest.skip("needs hipcc")
+    src, asm = tmp_path / "probe.hip", tmp_path / "probe.s"
+    src.write_text(_DMA_PROBE)
+    include = Path(build_hip.CSRC)
+    subprocess.run([build_hip.HIPCC, *build_hip.FLAGS, "--cuda-device-only", "-S", f"-I{include}",
+                    f"-I{include.parents[1] / 'include'}", str(src), "-o", str(asm)], check=True, capture_output=True)
+    lines = [line.strip() for line in asm.read_text().splitlines()]
+    lines = [line for line in lines if line.startswith((";;#ASM", "s_", "v_", "buffer_"))]
+    dma = [i for i, line in enumerate(lines) if re.match(r"buffer_load_dword.* lds$", line)]
+    assert len(dma) == 4, lines
+    begin = max(i for i in range(dma[1]) if lines[i].startswith(";;#ASMSTART"))
+    states = 0  # an instruction each, s_nop as many as it says
+    for line in lines[begin + 1:dma[1]]:
+        nop = re.match(r"s_nop (\d+)", line)
+        states += int(nop.group(1)) + 1 if nop else 1
+    assert states >= 5, lines[begin:dma[1] + 1]
+    # m0 goes to a register before the DMA's base does into it, and comes back from there
+    kept = re.match(r"s_mov_b32 (s\d+), m0$", lines[begin + 1])
+    assert kept and f"s_mov_b32 m0, {kept.group(1)}" in lines[dma[2] + 1:dma[3]], lines[begin:dma[3] + 1]
+    assert not any(re.search(rf"\b{kept.group(1)}\b", line) for line in lines[begin + 2:dma[2] + 1])
