@@ -34,6 +34,7 @@
 // staged through registers into a padded K tile and a transposed V tile,
 // double-buffered, the next chunk fetched while the current one computes).
 #include "spr_common.h"
+#include "spr_tile_order.h"
 #include <mutex>
 #include <type_traits>
 
@@ -177,14 +178,20 @@ __host__ __device__ inline int64_t plan_words(int32_t qn, int32_t kn) {
   return plan_seg_offset(qn) + 2 * (int64_t)qn * kn + 2 * (int64_t)qn + 2;
 }
 
-// Plan header (5 words after the bh_kv per-head plans): magic, bh_kv, qn, kn, s.  The plan kernels
+// After the bh_kv per-head plans: head_order[bh_kv], the kv heads by decreasing work (see
+// attn_tile_order_kernel), then the plan header.
+__host__ __device__ inline int32_t* head_order_at(int32_t* base, int64_t bh_kv, int32_t qn, int32_t kn) {
+  return base + bh_kv * plan_words(qn, kn);
+}
+
+// Plan header (5 words after head_order): magic, bh_kv, qn, kn, s.  The plan kernels
 // write it last; the attention kernels compare it with their own arguments and do
 // nothing when it does not match, so a plan built for other sizes (or never built)
 // cannot send them past the ends of the plan, Q or K/V.
 constexpr int32_t PLAN_MAGIC = 0x50525053;  // "SPRP"
 constexpr int PLAN_HEADER_WORDS = 5;
 __host__ __device__ inline int32_t* plan_header_at(int32_t* base, int64_t bh_kv, int32_t qn, int32_t kn) {
-  return base + bh_kv * plan_words(qn, kn);
+  return head_order_at(base, bh_kv, qn, kn) + bh_kv;
 }
 __device__ inline bool plan_matches(const int32_t* base, int64_t bh_kv, int32_t qn, int32_t kn, int32_t s) {
   const int32_t* hd = plan_header_at(const_cast<int32_t*>(base), bh_kv, qn, kn);
@@ -800,17 +807,11 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint8_t* p) {
 // and four LDS buffers rotate: chunk x is DMA'd right after the barrier of
 // chunk x - 3 (its buffer's previous chunk, x - 4, was last read before it)
 // and waited for before the barrier of chunk x - 1, two chunks later.
-constexpr int TILE_RUN = 8;  // consecutive tiles of a head on one XCD
-// turns of TILE_RUN tiles to each of the 8 XCDs that cover a head's tiles
-__host__ __device__ inline int32_t tile_turns(int64_t tiles) {
-  return static_cast<int32_t>((tiles + 8 * TILE_RUN - 1) / (8 * TILE_RUN));
-}
-
 template <bool KIDX, bool F16>
 __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int32_t s_q,
     int32_t s_kv, int32_t group, int32_t qn, int32_t kn, const int32_t* __restrict__ plan, int32_t bh_q,
-    int32_t tiles_per_head, float scale_log2, const int32_t* __restrict__ q_index,
+    spr::TileOrder order, float scale_log2, const int32_t* __restrict__ q_index,
     const int32_t* __restrict__ k_index, uint16_t* __restrict__ out, float* __restrict__ lse) {
   constexpr int NW = 8;
   constexpr int D = 128;
@@ -835,26 +836,17 @@ __global__ __launch_bounds__(512, 1) void attn_pipe_kernel(
   const int col = lane & 31;
   const int half = lane >> 5;
 
-  // ---- work item: workgroup b runs on XCD b % 8.  The heads follow one another and every
-  // head's 256-row tiles go to the XCDs in turn, TILE_RUN at a time, the first XCD moving on by
-  // one per head: the XCDs end together whatever the number of heads, all of them read the
-  // same head's keys (61 MB at 118,800 tokens, which the 256 MB last-level cache holds; eight
-  // heads it does not), and the tiles of a q-cluster mostly share an L2.  Against whole heads
-  // dealt to XCDs: 5 heads of 40,000 tokens (64 x 300 clusters, density 0.2) 1.09 -> 0.99 ms,
-  // 24 heads of 119,056 (302 x 1,002, density 0.22) 45.5 -> 42.5 ms, the 24 x 118,800-token
-  // layer 36.9 ms on both.  Runs of 2 instead of 8 cost that layer 1.5 %, of 4 0.5 %.
-  const int32_t per_head = tile_turns(tiles_per_head) * TILE_RUN;
-  const int64_t seq = blockIdx.x / 8;
-  const int64_t bhq = seq / per_head;
-  const int32_t in_head = static_cast<int32_t>(seq - bhq * per_head);
-  const int32_t xcd = static_cast<int32_t>((blockIdx.x + bhq) % 8);
-  const int32_t tile = (in_head / TILE_RUN * 8 + xcd) * TILE_RUN + in_head % TILE_RUN;
+  // ---- work item
+  int64_t slot;
+  int32_t tile;
+  order.at(blockIdx.x, slot, tile);
   if (!plan_matches(plan, bh_q / group, qn, kn, s_q)) {
     fill_nan_output(out, lse, bh_q, s_q, D, nan_pair<F16>());
     return;
   }
-  if (bhq >= bh_q) return;
-  const int64_t bhkv = bhq / group;
+  if (slot >= bh_q) return;
+  const int64_t bhkv = head_order_at(const_cast<int32_t*>(plan), bh_q / group, qn, kn)[slot / group];
+  const int64_t bhq = bhkv * group + slot % group;
   PlanView pv = plan_at(const_cast<int32_t*>(plan), bhkv, qn, kn);
   // tiles of a head in decreasing q-cluster key count (the plan's tile2_sorted order)
   if (tile >= pv.tile2_sorted[qn]) return;
@@ -1359,9 +1351,47 @@ constexpr int TO_MAX_QN = 4096;  // q-clusters per head the tile order handles i
 // workgroup per kv head; key counts, tile counts and the order staged in LDS.  The first
 // workgroup also writes the plan's header: a run launched after this kernel in stream order
 // sees the finished plan with it.
+//
+// One more workgroup orders the heads by decreasing work, sum over q-clusters of 256-row tiles x
+// 64-key chunks (ties by index): the heads follow one another over the tile grid, and a call
+// should end on a light one (16 heads of 35,400 tokens whose densities differ by up to 4: 2.81 ms
+// in index order, 2.69 so).  Identity where the terms are many: above HO_MAX heads or
+// HO_TERMS (head, q-cluster) pairs it would take longer than the others, and a call of so many
+// heads ends evenly.
+constexpr int HO_MAX = 1024;
+constexpr int HO_TERMS = 32768;
+__device__ void write_head_order(int32_t* plan, int32_t bh_kv, int32_t qn, int32_t kn) {
+  __shared__ unsigned long long work[HO_MAX];
+  int32_t* order = head_order_at(plan, bh_kv, qn, kn);
+  const int tid = threadIdx.x;
+  if (bh_kv > HO_MAX || static_cast<int64_t>(bh_kv) * qn > HO_TERMS) {
+    for (int h = tid; h < bh_kv; h += blockDim.x) order[h] = h;
+    return;
+  }
+  for (int h = tid; h < bh_kv; h += blockDim.x) work[h] = 0;
+  __syncthreads();
+  // terms spread over the workgroup, summed with LDS atomics (integers: any order)
+  for (int i = tid; i < bh_kv * qn; i += blockDim.x) {
+    const int h = i / qn, qc = i % qn;
+    const PlanView pv = plan_at(plan, h, qn, kn);
+    const int64_t w = static_cast<int64_t>(pv.tile2_off[qc + 1] - pv.tile2_off[qc]) * ((pv.total[qc] + BN - 1) / BN);
+    if (w != 0) atomicAdd(&work[h], static_cast<unsigned long long>(w));
+  }
+  __syncthreads();
+  for (int h = tid; h < bh_kv; h += blockDim.x) {
+    int rank = 0;
+    for (int o = 0; o < bh_kv; ++o) rank += (work[o] > work[h] || (work[o] == work[h] && o < h)) ? 1 : 0;
+    order[rank] = h;
+  }
+}
 __global__ __launch_bounds__(256) void attn_tile_order_kernel(int32_t* __restrict__ plan, int32_t qn, int32_t kn,
                                                               int32_t s) {
   extern __shared__ int32_t to_lds[];  // total[qn], tiles[qn], by_len[qn]
+  const int32_t bh_kv = static_cast<int32_t>(gridDim.x) - 1;
+  if (static_cast<int32_t>(blockIdx.x) == bh_kv) {
+    write_head_order(plan, bh_kv, qn, kn);
+    return;
+  }
   int32_t* tl = to_lds;
   int32_t* tc = to_lds + qn;
   int32_t* by_len = to_lds + 2 * qn;
@@ -1395,7 +1425,6 @@ __global__ __launch_bounds__(256) void attn_tile_order_kernel(int32_t* __restric
     }
     if (tid == 0) pv.tile2_sorted[qn] = run;
   } else if (tid == 64 && blockIdx.x == 0) {
-    const int32_t bh_kv = static_cast<int32_t>(gridDim.x);
     int32_t* hd = plan_header_at(plan, bh_kv, qn, kn);
     hd[0] = PLAN_MAGIC;
     hd[1] = bh_kv;
@@ -1406,7 +1435,7 @@ __global__ __launch_bounds__(256) void attn_tile_order_kernel(int32_t* __restric
 }
 
 extern "C" size_t spr_block_sparse_attention_workspace(int64_t bh_kv, int32_t qn, int32_t kn) {
-  return static_cast<size_t>((bh_kv * plan_words(qn, kn) + PLAN_HEADER_WORDS) * 4);
+  return static_cast<size_t>((bh_kv * plan_words(qn, kn) + bh_kv + PLAN_HEADER_WORDS) * 4);
 }
 
 // Plan for spr_block_sparse_attention_run: map uint8 [bh_kv, qn, kn], q_sizes
@@ -1445,7 +1474,7 @@ static int block_sparse_plan(const uint8_t* map, const int32_t* ids, const int32
   attn_plan_kernel<<<dim3(static_cast<uint32_t>(bh_kv), row_groups), THREADS, koff_bytes, stream>>>(
       map, ids, counts, q_sizes, k_sizes, qn, kn, static_cast<int32_t>(s), static_cast<int32_t*>(plan));
   SPR_LAUNCHED("attn_plan_kernel");
-  attn_tile_order_kernel<<<dim3(static_cast<uint32_t>(bh_kv)), 256, 3 * qn * sizeof(int32_t), stream>>>(
+  attn_tile_order_kernel<<<dim3(static_cast<uint32_t>(bh_kv) + 1), 256, 3 * qn * sizeof(int32_t), stream>>>(
       static_cast<int32_t*>(plan), qn, kn, static_cast<int32_t>(s));
   SPR_LAUNCHED("attn_tile_order_kernel");
   return SPR_OK;
@@ -1523,14 +1552,13 @@ extern "C" int spr_block_sparse_attention_run_ex(const void* q, const void* k, c
   uint16_t* o16 = static_cast<uint16_t*>(out);
   const int32_t s32 = static_cast<int32_t>(s), bhq32 = static_cast<int32_t>(bh_q);
   if (d == 128) {
-    const int64_t max_tiles_pipe = spr::ceil_div(s, 2 * BM) + qn;
-    const int64_t pipe_blocks = static_cast<int64_t>(tile_turns(max_tiles_pipe)) * TILE_RUN * 8 * bh_q;
-    SPR_REQUIRE(pipe_blocks < (int64_t(1) << 31), "spr_block_sparse_attention_run: too many tiles");
-    dim3 grid_pipe(static_cast<uint32_t>(pipe_blocks));
-    const int32_t tph = static_cast<int32_t>(max_tiles_pipe);
+    const int64_t row_tiles = spr::ceil_div(s, 2 * BM);
+    const spr::TileOrder order = spr::TileOrder::make(row_tiles, row_tiles + qn, bh_q);
+    SPR_REQUIRE(order.groups < (int64_t(1) << 31), "spr_block_sparse_attention_run: too many tiles");
+    dim3 grid_pipe(static_cast<uint32_t>(order.groups));
     auto pipe = [&](auto kxc, auto f) {
       attn_pipe_kernel<decltype(kxc)::value, decltype(f)::value><<<grid_pipe, 512, 0, stream>>>(
-          q16, k16, v16, s32, s32, group, qn, kn, pl, bhq32, tph, scale_log2, q_index, k_index, o16, lse);
+          q16, k16, v16, s32, s32, group, qn, kn, pl, bhq32, order, scale_log2, q_index, k_index, o16, lse);
     };
     using T_ = std::true_type;
     using F_ = std::false_type;

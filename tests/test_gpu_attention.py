@@ -88,10 +88,12 @@ def test_block_sparse_matches_closed_form(dev, oracle, B, Hq, Hkv, S, D, qn, kn)
 
 
 @pytest.mark.parametrize("Hq,Hkv,qn,D", [(1, 1, 1, 128), (3, 3, 7, 128), (10, 5, 8, 128), (9, 9, 17, 64),
-                                          (11, 11, 33, 128), (2, 2, 65, 128)])
+                                          (11, 11, 33, 128), (2, 2, 65, 128), (1025, 1025, 2, 128),
+                                          (6, 3, 140, 128)])
 def test_tile_order_reaches_every_tile(dev, oracle, Hq, Hkv, qn, D):
-    """Tile counts around the 8 tiles of a run and the 64 of one turn over the XCDs, head counts that leave the
-    last turn uneven: every row of every head is written once, by its own tile."""
+    """Tile counts around a run and one turn over the XCDs, head counts that leave the last turn uneven, more heads
+    than are put in order, tiles of both parts of the order: every row of every head is written once, by its own
+    tile."""
     from sparsepr_amd.kmeans_utils import dynamic_block_sparse_fwd_flashinfer
 
     rng = np.random.default_rng(100 * Hq + qn)

@@ -7,6 +7,7 @@ import shutil
 import subprocess
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 
@@ -89,3 +90,73 @@ def test_inline_dma_states_what_it_reads_and_writes(tmp_path):
     kept = re.match(r"s_mov_b32 (s\d+), m0$", lines[begin + 1])
     assert kept and f"s_mov_b32 m0, {kept.group(1)}" in lines[dma[2] + 1:dma[3]], lines[begin:dma[3] + 1]
     assert not any(re.search(rf"\b{kept.group(1)}\b", line) for line in lines[begin + 2:dma[2] + 1])
+
+
+_ORDER_PROBE = """
+#include <cstdio>
+#include <cstdlib>
+#include <hip/hip_runtime.h>
+#include "spr_tile_order.h"
+int main(int argc, char** argv) {
+  for (int i = 1; i + 2 < argc; i += 3) {
+    const spr::TileOrder o = spr::TileOrder::make(atoll(argv[i]), atoll(argv[i + 1]), atoll(argv[i + 2]));
+    printf("%lld", static_cast<long long>(o.groups));
+    for (int64_t b = 0; b < o.groups; ++b) {
+      int64_t head;
+      int32_t tile;
+      o.at(static_cast<uint32_t>(b), head, tile);
+      printf(" %lld %d", static_cast<long long>(head), tile);
+    }
+    printf("\\n");
+  }
+}
+"""
+
+
+def _tile_orders(tmp_path, calls):
+    """Per (row tiles, most tiles, heads): the (head, tile) of each workgroup, [groups, 2]."""
+    from sparsepr_amd import build_hip
+
+    if shutil.which(build_hip.HIPCC) is None:
+        pytest.skip("needs hipcc")
+    src, exe = tmp_path / "order.cpp", tmp_path / "order"
+    src.write_text(_ORDER_PROBE)
+    subprocess.run([build_hip.HIPCC, "-std=c++17", "-O1", "-x", "hip", "--offload-host-only",
+                    f"-I{build_hip.CSRC}", str(src), "-o", str(exe)], check=True, capture_output=True)
+    out = subprocess.run([str(exe), *(str(v) for call in calls for v in call)], check=True, capture_output=True)
+    rows = [np.array(line.split(), dtype=np.int64) for line in out.stdout.decode().splitlines()]
+    assert all(len(r) == 1 + 2 * r[0] for r in rows)
+    return [r[1:].reshape(-1, 2) for r in rows]
+
+
+def test_tile_order_deals_every_tile_once_and_the_longest_early(tmp_path):
+    """Every tile of every head has one workgroup, with few to spare, and list scheduling on 8 XCDs
+    of 32 workgroups ends near the ideal: with a prompt, whose query tiles keep every key and so walk
+    1 / density = 5 times the chunks, and without one."""
+    edges = [(rows, most, heads) for rows, most in ((1, 2), (7, 9), (16, 17), (79, 130), (80, 81), (465, 765))
+             for heads in (1, 2, 7, 8, 9, 24, 300)]
+    for (rows, most, heads), order in zip(edges, _tile_orders(tmp_path, edges)):
+        got = order[(order[:, 0] < heads) & (order[:, 1] < most)]
+        assert len(got) == heads * most and len(np.unique(got, axis=0)) == heads * most
+        run = 8 if rows >= 256 else 4 if rows >= 32 else 2
+        assert len(order) <= heads * (most + 4 * run) + 16 * run  # two parts, each an odd number of runs
+    rng = np.random.default_rng(0)
+    cases = [(heads, tokens, text) for heads in (3, 5, 8, 12, 16, 24) for tokens in (20000, 35400, 60000, 118800)
+             for text in (0, 256, 512)]
+    calls = [(-(-(n + text) // 256), -(-(n + text) // 256) + n // 400, h) for h, n, text in cases]
+    for (heads, tokens, text), call, order in zip(cases, calls, _tile_orders(tmp_path, calls)):
+        ordinary = tokens // 5 // 64
+        cost = np.zeros((heads, call[1]))
+        for h in range(heads):
+            live = -(-tokens // 256) + tokens // 800
+            cost[h, :live] = np.sort(ordinary * rng.uniform(0.8, 1.1, live))[::-1]
+            if text:
+                cost[h, :live + 2] = np.concatenate(([5 * ordinary] * 2, cost[h, :live]))
+        ends = np.zeros((8, 32))
+        for b, (h, tile) in enumerate(order):
+            if h < heads and tile < call[1]:
+                xcd = ends[b % 8]
+                xcd[xcd.argmin()] += cost[h, tile]
+        # at most an ordinary tile and a half after the ideal end
+        excess = (ends.max() - max(cost.sum() / 256, cost.max())) / ordinary
+        assert excess <= 1.5, (heads, tokens, text, excess)
