@@ -16,7 +16,8 @@
 //       score = log(max(E / n_c, 1e-30)) + 2 m;  -inf for an empty cluster
 //   attention mass: score = log(max(sum_t e^(l_t - m), 1e-30)) + m, m = max_t l_t
 // The weights are taken against a reference that starts at l_c (the mass: at the first
-// chunk's maximum) and moves only when a logit passes it by SE_SLACK, with the sums rescaled;
+// chunk's maximum) and moves only when a logit passes it by SE_SLACK (less where |v|^2 is large),
+// with the sums rescaled;
 // the scores do not depend on it but for rounding.
 //
 // Layout.  A first kernel writes the centroid logits l_c [query head, centroid, cluster]
@@ -85,13 +86,6 @@ __device__ __forceinline__ float dpp_mov(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 
-// sum over lanes 8 i .. 8 i + 7 (quad_perm [1, 0, 3, 2], [2, 3, 0, 1], then row_half_mirror)
-__device__ __forceinline__ float oct_sum(float v) {
-  v += dpp_mov<0xB1>(v);
-  v += dpp_mov<0x4E>(v);
-  return v + dpp_mov<0x141>(v);
-}
-
 // max / sum over lanes l and l ^ 32: v_permlane32_swap of x with itself gives the
 // lower half-wave's value in the first result and the upper half's in the second on
 // every lane, so both lanes of a pair combine the same two operands in the same order.
@@ -102,6 +96,17 @@ __device__ __forceinline__ float max_xor32(float x) {
 __device__ __forceinline__ float sum_xor32(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// max over the wave: quad_perm [1, 0, 3, 2] and [2, 3, 0, 1], row_half_mirror and row_mirror give
+// each lane its row of 16, the swaps the four rows
+__device__ __forceinline__ float wave_max(float x) {
+  x = fmaxf(x, dpp_mov<0xB1>(x));
+  x = fmaxf(x, dpp_mov<0x4E>(x));
+  x = fmaxf(x, dpp_mov<0x141>(x));
+  x = fmaxf(x, dpp_mov<0x140>(x));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return max_xor32(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
 }
 
 constexpr int SE_ROW = SE_D * 2;  // bytes per bf16 token row
@@ -194,9 +199,11 @@ constexpr int SE_SWAVES = 2;  // waves that take the V statistics, every other c
 constexpr int SE_TILES = 8;   // chunks of K in LDS
 constexpr int SE_VTILES = 6;  // chunks of V, whose statistics are taken a step ahead
 constexpr int SE_TILE = SE_CHUNK * SE_ROW;  // bytes of a K or V tile
-// a running reference is moved once a chunk's largest logit passes it by this much: the weights
-// stay below e^30, their squares times a cluster's values inside fp32
+// A running reference is moved once a chunk's largest logit passes it by this much, or by less
+// where the squared weights times the chunk's largest |v|^2, over all the cluster's tokens, would
+// pass SE_TOP: whatever the values, the sums are finite where they are against the largest logit.
 constexpr float SE_SLACK = 30.0f;
+constexpr float SE_TOP = 1.0e37f;
 
 template <int MODE>  // 0: value error (scores holds l_c on entry), 1: attention mass
 __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score_kernel(
@@ -209,6 +216,7 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
   __shared__ __attribute__((aligned(16))) uint16_t vc_l[MODE == 0 ? 3 * SE_CPW + 1 : 1][SE_D];
   __shared__ __attribute__((aligned(16))) float vn_l[4][SE_CHUNK];  // |v_t|^2
   __shared__ __attribute__((aligned(16))) float cd_l[4][SE_CHUNK];  // -2 v_t . vc
+  __shared__ float slack_l[4];  // the chunk's: at most SE_SLACK
   __shared__ float vc2_l[SE_CPW];
   // per cluster and row of a q wave: the sum, the reference it is taken against, the largest logit
   __shared__ float es_l[SE_CPW][32 * SE_QWAVES];
@@ -343,7 +351,7 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
   };
   // |v_t|^2 (the diagonal of V V^T) and -2 v_t . vc (V against the three pieces of vc in
   // columns 0 .. 2) of a chunk: exact products, fp32 sums
-  auto vstats = [&](int j, const uint8_t* vt, int buf) {
+  auto vstats = [&](int j, int len, const uint8_t* vt, int buf) {
     f32x16 vv = f32x16{}, vc = f32x16{};
     const uint16_t* brow = vc_l[col < 3 ? 3 * j + col : 3 * SE_CPW] + 8 * half;
 #pragma unroll
@@ -356,7 +364,14 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
     float diag = 0.0f;  // row col is element 4 (col / 8) + col % 4 of the half with bit 2 of col
 #pragma unroll
     for (int e = 0; e < 16; ++e) diag = e == 4 * (col >> 3) + (col & 3) ? vv[e] : diag;
-    if (half == ((col >> 2) & 1)) vn_l[buf][col] = diag;
+    const bool mine = half == ((col >> 2) & 1);
+    if (mine) vn_l[buf][col] = diag;
+    // rows of the next cluster may be among them: the slack is then shorter than it has to be
+    const float vmax = wave_max(mine ? diag : 0.0f);
+    if (lane == 0) {
+      const float room = 0.5f * (logf(SE_TOP / static_cast<float>(len)) - logf(vmax));
+      slack_l[buf] = fminf(fmaxf(room, 0.0f), SE_SLACK);
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       f32x4 c;
@@ -441,7 +456,7 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
     // S^T of a chunk (16 MFMAs), folded into the state:
     // E = sum_t max(c_w^2 |vc|^2 + r (r |v|^2 - 2 c_w v.vc), 0) with r = e^(l_t - ref),
     // c_w = e^(l_c - ref).  ref starts at l_c (c_w = 1: no product per element) and moves only
-    // when a logit passes it by SE_SLACK; the result does not depend on it but for rounding.
+    // when a logit passes it by the chunk's slack; the result does not depend on it but for rounding.
     auto fold = [&](auto masked, const uint8_t* kt, int buf, int cn, int jc) {
       constexpr bool MASKED = decltype(masked)::value;
       f32x16 cur;
@@ -459,7 +474,7 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
       // max over the raw dot products, scaled once: fl(a s) is monotone in a for s > 0
       cmax = max_xor32(cmax) * scale;
       top = fmaxf(top, cmax);
-      const bool up = cmax > ref + SE_SLACK;
+      const bool up = cmax > ref + (MODE == 0 ? slack_l[buf] : SE_SLACK);
       if (__ballot(up) != 0ull) {
         const float to = up ? cmax : ref;
         const float alpha = up ? exp_fast(ref - to) : 1.0f;
@@ -532,7 +547,7 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         if (inside(wn)) {
-          if (i == stat) vstats(wn.j, v_tiles + taken % SE_VTILES * SE_TILE, taken & 3);
+          if (i == stat) vstats(wn.j, wn.len, v_tiles + taken % SE_VTILES * SE_TILE, taken & 3);
           ++taken;
           advance(wn);
         }
@@ -775,7 +790,7 @@ extern "C" int spr_svg_ear_scores(const float* q_centroids, const uint16_t* k_so
                 "spr_svg_ear_scores: Jensen-aware routing requires var_k_diag");
   }
   // Query blocks of 32 rows, one wave each, in groups of equal size of at most SE_QWAVES; up to
-  // five blocks get two waves each.  One more wave takes the V statistics, and four move the tiles.
+  // five blocks get two waves each.  Two more take the V statistics, and four of all move the tiles.
   const int32_t qblocks = (qn + 31) / 32;
   const int32_t qgroups = (qblocks + SE_QWAVES - 1) / SE_QWAVES;
   const int32_t qwaves = (qblocks + qgroups - 1) / qgroups;

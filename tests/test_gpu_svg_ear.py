@@ -110,6 +110,30 @@ def test_scores_at_the_edges_of_the_wave_split(dev, oracle, qn, kn, qscale):
         assert (np.abs(a[fin] - ref[fin]) <= ATOL + 1e-5 * np.abs(ref[fin])).all()
 
 
+@pytest.mark.parametrize("vscale", [1e-10, 1e8, 1e16])
+@pytest.mark.parametrize("qn", [40, 161])
+def test_value_error_scores_hold_for_large_and_small_values(dev, oracle, vscale, qn):
+    """Logits 4 to 28 above the centroid's with |v|^2 up to 1e34, whose products with weights taken
+    against the centroid's logit pass fp32 though those against the largest logit do not, and with
+    |v|^2 near the 1e-30 under which a score is clamped.  The bound is 2e-3 and 1e-5 of the score."""
+    from sparsepr_amd.kernels.svg_ear import svg_ear_value_error_scores_triton
+
+    sizes = np.array([[33, 5, 64, 100, 1]], np.int32)
+    qc, k, v, kc, vc, _ = _case(qn, 1, 1, qn, sizes)
+    qc = np.abs(qc)
+    top = np.linspace(4.0, 28.0, k.shape[1], dtype=np.float32)[None, :, None]
+    k = _bf16_np(oracle, (0.1 * k + top * np.sqrt(128.0) / qc.mean(axis=1).sum()).astype(np.float32))
+    v = _bf16_np(oracle, (v * vscale * np.array([1.0, 1e-3])[np.arange(v.shape[1]) % 2][None, :, None]).astype(np.float32))
+    kc, vc = 0.0 * kc, (vc * vscale).astype(np.float32)
+    got = svg_ear_value_error_scores_triton(
+        qcentroids=to_dev(qc, dev), k_sorted=to_dev(k, dev, torch.bfloat16), v_sorted=to_dev(v, dev, torch.bfloat16),
+        kcentroids=to_dev(kc, dev), vcentroids=to_dev(vc, dev), kcluster_sizes=to_dev(sizes, dev), gqa_group=1)
+    ref = oracle.svg_ear_value_error_scores(qc, k, v, kc, vc, sizes, 1)
+    got = got.cpu().numpy().astype(np.float64)
+    assert np.isfinite(ref).all() and np.isfinite(got).all()
+    assert (np.abs(got - ref) <= ATOL + 1e-5 * np.abs(ref)).all()
+
+
 def test_grouped_scores_equal_ungrouped(dev, oracle):
     from sparsepr_amd.kernels.svg_ear import (svg_ear_grouped_value_error_scores_triton,
                                               svg_ear_value_error_scores_triton)
