@@ -26,10 +26,11 @@
 // workgroup per CU for (query head, 8 consecutive key clusters, up to 320 query rows): a wave
 // per 32-row query block (two for up to five blocks, each folding every other chunk), two
 // waves for the statistics of V, at most twelve, three per SIMD.  K and V are walked once for
-// all rows.  The clusters' tokens are one contiguous run, walked in 32-token chunks (a chunk
+// all rows.  Calls of up to 128 rows with many short clusters take four waves, one chunk per
+// barrier and half the LDS, two workgroups per CU (the host's rule).  The clusters' tokens are one contiguous run, walked in 32-token chunks (a chunk
 // never spans two clusters), whose K and V rows are DMA'd into swizzled LDS tiles (16-byte
 // piece p of token row t at slot p ^ (t % 16): the MFMA fragment reads hit 16 distinct slots
-// per 16 lanes) two steps of two chunks ahead.  A query wave forms S^T = K Q~^T by 16 bf16
+// per 16 lanes) two steps ahead.  A query wave forms S^T = K Q~^T by 16 bf16
 // MFMAs per chunk: q~ is split into bf16 hi + lo with hi + lo == q~ exactly (q~ has 11
 // significant bits, hi the top 8, lo the next 3), so every product is the reference's TF32
 // product exactly and only the fp32 summation order differs.  |v_t|^2 and v_t . vc are products
@@ -192,38 +193,42 @@ __global__ __launch_bounds__(SE_THREADS) void svg_ear_centroid_logit_kernel(
   if (r1 < qn) store(r1, dot1, s21);
 }
 
-// Key clusters per workgroup and the most query waves of one.
-constexpr int SE_CPW = 8;
-constexpr int SE_QWAVES = 10;
-constexpr int SE_SWAVES = 2;  // waves that take the V statistics, every other chunk each
-constexpr int SE_TILES = 8;   // chunks of K in LDS
-constexpr int SE_VTILES = 6;  // chunks of V, whose statistics are taken a step ahead
+constexpr int SE_CPW = 8;     // key clusters per workgroup
+constexpr int SE_SWAVES = 2;  // waves that take the V statistics
+// A workgroup of the score kernel walks STEP chunks per barrier.
+template <int STEP>
+struct Step {
+  static constexpr int QWAVES = STEP == 2 ? 10 : 4;  // the most query waves
+  static constexpr int TILES = 4 * STEP;             // chunks of K in LDS
+  static constexpr int VTILES = 3 * STEP;            // chunks of V, whose statistics are taken a step ahead
+  static constexpr int STATS = 2 * STEP;             // chunks whose statistics are kept
+};
 constexpr int SE_TILE = SE_CHUNK * SE_ROW;  // bytes of a K or V tile
 // A running reference is moved once a chunk's largest logit passes it by this much, or by less
 // where the squared weights times the chunk's largest |v|^2, over all the cluster's tokens, would
-// pass SE_TOP: whatever the values, the sums are finite where they are against the largest logit.
+// pass 2^123: whatever the values, the sums are finite where they are against the largest logit.
 constexpr float SE_SLACK = 30.0f;
-constexpr float SE_TOP = 1.0e37f;
 
-template <int MODE>  // 0: value error (scores holds l_c on entry), 1: attention mass
-__global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score_kernel(
+template <int MODE, int STEP>  // 0: value error (scores holds l_c on entry), 1: attention mass
+__global__ __launch_bounds__(64 * (STEP == 2 ? Step<2>::QWAVES + SE_SWAVES : 4), STEP == 2 ? 3 : 2) void svg_ear_score_kernel(
     const float* __restrict__ qc, const uint16_t* __restrict__ ks, const uint16_t* __restrict__ vs,
     const float* __restrict__ vcent, const int32_t* __restrict__ k_sizes, int32_t qn, int32_t kn, int64_t t_stored,
     int32_t group, int32_t qgroups, int32_t qwaves, int32_t sets, float* __restrict__ scores) {
-  __shared__ __attribute__((aligned(1024))) uint8_t k_tiles[SE_TILES * SE_TILE];
-  __shared__ __attribute__((aligned(1024))) uint8_t v_tiles[MODE == 0 ? SE_VTILES * SE_TILE : 16];
+  using S = Step<STEP>;
+  __shared__ __attribute__((aligned(1024))) uint8_t k_tiles[S::TILES * SE_TILE];
+  __shared__ __attribute__((aligned(1024))) uint8_t v_tiles[MODE == 0 ? S::VTILES * SE_TILE : 16];
   // the value centroids as three bf16 pieces whose sum they are, and a row of zeros
   __shared__ __attribute__((aligned(16))) uint16_t vc_l[MODE == 0 ? 3 * SE_CPW + 1 : 1][SE_D];
-  __shared__ __attribute__((aligned(16))) float vn_l[4][SE_CHUNK];  // |v_t|^2
-  __shared__ __attribute__((aligned(16))) float cd_l[4][SE_CHUNK];  // -2 v_t . vc
-  __shared__ float slack_l[4];  // the chunk's: at most SE_SLACK
+  __shared__ __attribute__((aligned(16))) float vn_l[S::STATS][SE_CHUNK];  // |v_t|^2
+  __shared__ __attribute__((aligned(16))) float cd_l[S::STATS][SE_CHUNK];  // -2 v_t . vc
+  __shared__ float slack_l[S::STATS][2];  // the chunk's, the less of the two: at most SE_SLACK
   __shared__ float vc2_l[SE_CPW];
   // per cluster and row of a q wave: the sum, the reference it is taken against, the largest logit
-  __shared__ float es_l[SE_CPW][32 * SE_QWAVES];
-  __shared__ float rf_l[SE_CPW][32 * SE_QWAVES];
-  __shared__ float tp_l[SE_CPW][32 * SE_QWAVES];
+  __shared__ float es_l[SE_CPW][32 * S::QWAVES];
+  __shared__ float rf_l[SE_CPW][32 * S::QWAVES];
+  __shared__ float tp_l[SE_CPW][32 * S::QWAVES];
   __shared__ int32_t len_l[SE_CPW];  // tokens in each run (clamped)
-  __shared__ int64_t red_l[SE_QWAVES + SE_SWAVES];
+  __shared__ int64_t red_l[S::QWAVES + SE_SWAVES];
 
   // Workgroup b runs on XCD b % 8: the query groups of the same clusters follow one another
   // there and find K and V in its L2.
@@ -246,7 +251,11 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
   const int set = wave / qwaves;
   const int q = q0 + 32 * (wave % qwaves) + col;
   const bool q_wave = set < sets && q0 + 32 * (wave % qwaves) < qn;
-  const int stat = MODE == 0 ? wave - qwaves * sets : -1;  // 0 or 1: takes the statistics of that chunk of a step
+  // Who takes the statistics of V: at STEP 2 two waves of their own (stat 0 and 1), a chunk of a
+  // step each; at STEP 1 waves 2 and 3, a half of every chunk's, or with three or four query waves
+  // all four, a quarter each.
+  const int stat = wave - qwaves * sets;
+  const bool quarters = STEP == 1 && qwaves > 2;
   const int rows = 32 * qwaves;
 
   // the query rows on their way while the rest is set up (rows past the end read the last one,
@@ -351,38 +360,76 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
   };
   // |v_t|^2 (the diagonal of V V^T) and -2 v_t . vc (V against the three pieces of vc in
   // columns 0 .. 2) of a chunk: exact products, fp32 sums
-  auto vstats = [&](int j, int len, const uint8_t* vt, int buf) {
+  // A chunk's slack from its |v|^2 (those of the next cluster's rows may be among them: it is then
+  // shorter than it has to be): half of ln(2^123 / (len max |v|^2)), less than SE_SLACK only where
+  // len |v|^2 passes 2^123 / e^60.  An overflowing product leaves none.
+  auto chunk_slack = [&](int len, float vn) {
+    const float sum = static_cast<float>(len) * vn;
+    if (__ballot(sum > 6.0e10f) == 0ull) return SE_SLACK;
+    return fminf(fmaxf(0.5f / SE_LOG2E * (123.0f - __builtin_amdgcn_logf(wave_max(sum))), 0.0f), SE_SLACK);
+  };
+  auto quad_sum3 = [&](float x) {  // columns 0 .. 3 (the last is zero) lie in one quad
+    x += dpp_mov<0xB1>(x);
+    return x + dpp_mov<0x4E>(x);
+  };
+  auto vstats = [&](auto norms, auto dots, int j, int len, const uint8_t* vt, int buf) {
+    constexpr bool NORMS = decltype(norms)::value, DOTS = decltype(dots)::value;
     f32x16 vv = f32x16{}, vc = f32x16{};
     const uint16_t* brow = vc_l[col < 3 ? 3 * j + col : 3 * SE_CPW] + 8 * half;
 #pragma unroll
     for (int s = 0; s < SE_KSTEPS; ++s) {
       const u32x4 a = tile_frag(vt, s);
-      const u32x4 b = *reinterpret_cast<const u32x4*>(brow + 16 * s);
-      vv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(spr::as_bf16x8(a), spr::as_bf16x8(a), vv, 0, 0, 0);
-      vc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(spr::as_bf16x8(a), spr::as_bf16x8(b), vc, 0, 0, 0);
+      if (NORMS) vv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(spr::as_bf16x8(a), spr::as_bf16x8(a), vv, 0, 0, 0);
+      if (DOTS) {
+        const u32x4 b = *reinterpret_cast<const u32x4*>(brow + 16 * s);
+        vc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(spr::as_bf16x8(a), spr::as_bf16x8(b), vc, 0, 0, 0);
+      }
     }
-    float diag = 0.0f;  // row col is element 4 (col / 8) + col % 4 of the half with bit 2 of col
+    if (NORMS) {
+      float diag = 0.0f;  // row col is element 4 (col / 8) + col % 4 of the half with bit 2 of col
 #pragma unroll
-    for (int e = 0; e < 16; ++e) diag = e == 4 * (col >> 3) + (col & 3) ? vv[e] : diag;
-    const bool mine = half == ((col >> 2) & 1);
-    if (mine) vn_l[buf][col] = diag;
-    // rows of the next cluster may be among them: the slack is then shorter than it has to be
-    const float vmax = wave_max(mine ? diag : 0.0f);
-    if (lane == 0) {
-      const float room = 0.5f * (logf(SE_TOP / static_cast<float>(len)) - logf(vmax));
-      slack_l[buf] = fminf(fmaxf(room, 0.0f), SE_SLACK);
+      for (int e = 0; e < 16; ++e) diag = e == 4 * (col >> 3) + (col & 3) ? vv[e] : diag;
+      const bool mine = half == ((col >> 2) & 1);
+      if (mine) vn_l[buf][col] = diag;
+      const float slack = chunk_slack(len, mine ? diag : 0.0f);
+      if (lane < 2) slack_l[buf][lane] = slack;
     }
+    if (DOTS) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < 4; ++i) {
+        f32x4 c;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c[r] = -2.0f * quad_sum3(vc[4 * i + r]);
+        if (col == 0) *reinterpret_cast<f32x4*>(&cd_l[buf][8 * i + 4 * half]) = c;
+      }
+    }
+  };
+  // A quarter of that by 16 x 16 blocks: |v_t|^2, or -2 v_t . vc, of the chunk's lower or upper 16
+  // tokens.
+  auto vstats_quarter = [&](int part, bool dots, int j, int len, const uint8_t* vt, int buf) {
+    const int c16 = lane & 15, g = lane >> 4, row = 16 * part + c16;
+    const uint16_t* brow = vc_l[c16 < 3 ? 3 * j + c16 : 3 * SE_CPW] + 8 * g;
+    f32x4 acc = f32x4{};
+#pragma unroll
+    for (int s = 0; s < SE_D / 32; ++s) {  // token row, dims 32 s + 8 g + 0 .. 7
+      const u32x4 a = *reinterpret_cast<const u32x4*>(vt + row * SE_ROW + (((4 * s + g) ^ c16) << 4));
+      const u32x4 b = dots ? *reinterpret_cast<const u32x4*>(brow + 32 * s) : a;
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(spr::as_bf16x8(a), spr::as_bf16x8(b), acc, 0, 0, 0);
+    }
+    // lane (column c16, g) holds rows 4 g + 0 .. 3
+    if (dots) {
       f32x4 c;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float x = vc[4 * i + r];  // columns 0 .. 3 (the last is zero) lie in one quad
-        x += dpp_mov<0xB1>(x);
-        x += dpp_mov<0x4E>(x);
-        c[r] = -2.0f * x;
-      }
-      if (col == 0) *reinterpret_cast<f32x4*>(&cd_l[buf][8 * i + 4 * half]) = c;
+      for (int r = 0; r < 4; ++r) c[r] = -2.0f * quad_sum3(acc[r]);
+      if (c16 == 0) *reinterpret_cast<f32x4*>(&cd_l[buf][16 * part + 4 * g]) = c;
+    } else {
+      float diag = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) diag = r == (c16 & 3) ? acc[r] : diag;
+      const bool mine = g == c16 >> 2;
+      if (mine) vn_l[buf][row] = diag;
+      const float slack = chunk_slack(len, mine ? diag : 0.0f);
+      if (lane == 0) slack_l[buf][part] = slack;
     }
   };
 
@@ -390,35 +437,56 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
   enter(wc, 0);
   wn = wd = wc;
   int folded = 0, taken = 0, issued = 0;  // how many of each so far
-  // Step p folds chunks 2 p and 2 p + 1 and takes the statistics of the two after them; two more
-  // are in flight and another two go to the tiles of the step before.  Two chunks to a barrier
-  // let the waves of a SIMD drift apart, one's MFMAs beside another's exponentials.  Every wave
-  // takes the same steps.
+  // Step p folds chunks STEP p .. + STEP - 1 and takes the statistics of the STEP after them; as
+  // many more are in flight and another STEP go to the tiles of the step before.  Every wave takes
+  // the same steps.
   auto issue = [&] {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < STEP; ++i) {
       if (inside(wd)) {
-        dma(wd, issued % SE_TILES * SE_TILE, issued % SE_VTILES * SE_TILE);
+        dma(wd, issued % S::TILES * SE_TILE, issued % S::VTILES * SE_TILE);
         ++issued;
         advance(wd);
       }
     }
   };
-  auto landed = [&](int upto) {  // chunks below `upto`, for every wave; two more may be in flight
-    if (issued >= upto + 2) spr::wait_vm<2 * DMA_PER_CHUNK>();
-    else if (issued == upto + 1) spr::wait_vm<DMA_PER_CHUNK>();
+  auto landed = [&](int upto) {  // chunks below `upto`, for every wave; STEP more may be in flight
+    if (issued >= upto + STEP) spr::wait_vm<STEP * DMA_PER_CHUNK>();
+    else if (STEP == 2 && issued == upto + 1) spr::wait_vm<DMA_PER_CHUNK>();
     else spr::wait_vm<0>();
     spr::lds_barrier();
   };
   auto first = [&] {
     issue();
     issue();
-    landed(2);
+    landed(STEP);
     issue();
   };
   auto begin_step = [&] {
-    landed(folded + 4);
+    landed(folded + 2 * STEP);
     issue();
+  };
+  auto stats = [&] {
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+#pragma unroll
+    for (int i = 0; i < STEP; ++i) {
+      if (inside(wn)) {
+        const uint8_t* vt = v_tiles + taken % S::VTILES * SE_TILE;
+        const int buf = taken % S::STATS;
+        if constexpr (STEP == 2) {
+          if (i == stat) vstats(yes, yes, wn.j, wn.len, vt, buf);
+        } else if (quarters) {
+          vstats_quarter(wave & 1, wave >= 2, wn.j, wn.len, vt, buf);
+        } else if (wave == 2) {
+          vstats(yes, no, wn.j, wn.len, vt, buf);
+        } else if (wave == 3) {
+          vstats(no, yes, wn.j, wn.len, vt, buf);
+        }
+        ++taken;
+        advance(wn);
+      }
+    }
   };
   if (q_wave) {
     // B fragments: q~ dims 16 s + 8 half + 0..7 as bf16 hi and lo, in registers before the
@@ -474,7 +542,7 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
       // max over the raw dot products, scaled once: fl(a s) is monotone in a for s > 0
       cmax = max_xor32(cmax) * scale;
       top = fmaxf(top, cmax);
-      const bool up = cmax > ref + (MODE == 0 ? slack_l[buf] : SE_SLACK);
+      const bool up = cmax > ref + (MODE == 0 ? fminf(slack_l[buf][0], slack_l[buf][1]) : SE_SLACK);
       if (__ballot(up) != 0ull) {
         const float to = up ? cmax : ref;
         const float alpha = up ? exp_fast(ref - to) : 1.0f;
@@ -512,10 +580,14 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
       }
       esum += add0 + add1;
     };
-    if (inside(wc)) first();
+    if (inside(wc)) {
+      first();
+      if (MODE == 0 && quarters) stats();
+    }
     while (inside(wc)) {
       begin_step();
-      for (int i = 0; i < 2 && inside(wc); ++i) {
+      if (MODE == 0 && quarters) stats();
+      for (int i = 0; i < STEP && inside(wc); ++i) {
         if (sets == 1 || i == set) {
           const int slot = set * rows + 32 * (wave % qwaves) + col;
           if (wc.c0 < sets * SE_CHUNK) {  // this wave's first chunk of the cluster
@@ -526,9 +598,9 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
             esum = 0.0f;
           }
           const int cn = min(SE_CHUNK, wc.len - wc.c0);
-          const uint8_t* kt = k_tiles + folded % SE_TILES * SE_TILE;
-          if (cn == SE_CHUNK) fold(std::false_type{}, kt, folded & 3, cn, wc.j);
-          else fold(std::true_type{}, kt, folded & 3, cn, wc.j);
+          const uint8_t* kt = k_tiles + folded % S::TILES * SE_TILE;
+          if (cn == SE_CHUNK) fold(std::false_type{}, kt, folded % S::STATS, cn, wc.j);
+          else fold(std::true_type{}, kt, folded % S::STATS, cn, wc.j);
           if (wc.c0 + sets * SE_CHUNK >= wc.len) {  // its last
             const float total = sum_xor32(esum);
             if (half == 0) {
@@ -543,24 +615,14 @@ __global__ __launch_bounds__((SE_QWAVES + SE_SWAVES) * 64, 3) void svg_ear_score
       }
     }
   } else {
-    auto stats = [&] {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        if (inside(wn)) {
-          if (i == stat) vstats(wn.j, wn.len, v_tiles + taken % SE_VTILES * SE_TILE, taken & 3);
-          ++taken;
-          advance(wn);
-        }
-      }
-    };
     if (inside(wc)) {
       first();
-      stats();
+      if constexpr (MODE == 0) stats();
     }
     while (inside(wc)) {
       begin_step();
-      stats();
-      for (int i = 0; i < 2 && inside(wc); ++i) {
+      if constexpr (MODE == 0) stats();
+      for (int i = 0; i < STEP && inside(wc); ++i) {
         ++folded;
         advance(wc);
       }
@@ -789,16 +851,25 @@ extern "C" int spr_svg_ear_scores(const float* q_centroids, const uint16_t* k_so
     SPR_REQUIRE(!(jensen_var_cap > 0.0f) || var_k_diag != nullptr,
                 "spr_svg_ear_scores: Jensen-aware routing requires var_k_diag");
   }
-  // Query blocks of 32 rows, one wave each, in groups of equal size of at most SE_QWAVES; up to
-  // five blocks get two waves each.  Two more take the V statistics, and four of all move the tiles.
+  // Query blocks of 32 rows, one wave each, in groups of equal size; four waves of all move the
+  // tiles.  Up to four blocks leave most of a CU idle: its workgroups then take half the LDS, so
+  // that two share it, where there are 1.5 or more for each CU and the clusters are short enough
+  // (in long ones the second chunk per barrier and the two sets of query waves are worth more).
+  // 24 heads x 40,000 tokens, 64 rows: 1,000 clusters 284 -> 216 us, 134 clusters 184 -> 180;
+  // 118,800 tokens, 134 clusters 440 -> 461.  128 rows: 1,000 clusters 331 -> 276 us, 300
+  // clusters 226 -> 230.  8 heads x 40,000 tokens (304 workgroups), 64 rows: 92 -> 98 us.
   const int32_t qblocks = (qn + 31) / 32;
-  const int32_t qgroups = (qblocks + SE_QWAVES - 1) / SE_QWAVES;
+  const int64_t cluster_tokens = mode == 0 && qblocks > 2 ? 128 : 512;  // mean of the longest that are short
+  const bool few = qblocks <= Step<1>::QWAVES && spr::ceil_div(kn, SE_CPW) * q_heads >= 384 &&
+                   t_stored <= cluster_tokens * kn;
+  const int32_t most = few ? Step<1>::QWAVES : Step<2>::QWAVES;
+  const int32_t qgroups = (qblocks + most - 1) / most;
   const int32_t qwaves = (qblocks + qgroups - 1) / qgroups;
-  const int32_t sets = 2 * qwaves <= SE_QWAVES ? 2 : 1;
+  const int32_t sets = !few && 2 * qwaves <= most ? 2 : 1;
   const int64_t turns = static_cast<int64_t>((kn + 8 * SE_CPW - 1) / (8 * SE_CPW)) * qgroups;
   SPR_REQUIRE(turns * 8 < (int64_t(1) << 31), "spr_svg_ear_scores: grid too large");
   const dim3 grid(static_cast<uint32_t>(turns * 8), static_cast<uint32_t>(q_heads));
-  const int32_t waves = qwaves * sets + (mode == 0 ? SE_SWAVES : 0);
+  const int32_t waves = qwaves * sets + (mode == 0 && !few ? SE_SWAVES : 0);
   const uint32_t threads = 64 * (waves < 4 ? 4 : waves);
   if (mode == 0) {
     const bool jensen = jensen_var_cap > 0.0f;
@@ -808,12 +879,18 @@ extern "C" int spr_svg_ear_scores(const float* q_centroids, const uint16_t* k_so
                                     SE_THREADS, 0, stream>>>(q_centroids, k_centroids, jensen ? var_k_diag : nullptr,
                                                              jensen ? jensen_var_cap : 0.0f, qn, kn, group, scores);
     SPR_LAUNCHED("svg_ear_centroid_logit_kernel");
-    svg_ear_score_kernel<0><<<grid, threads, 0, stream>>>(q_centroids, k_sorted, v_sorted, v_centroids, k_sizes, qn,
-                                                          kn, t_stored, group, qgroups, qwaves, sets, scores);
+    auto score = [&](auto step) {
+      svg_ear_score_kernel<0, decltype(step)::value><<<grid, threads, 0, stream>>>(
+          q_centroids, k_sorted, v_sorted, v_centroids, k_sizes, qn, kn, t_stored, group, qgroups, qwaves, sets, scores);
+    };
+    if (few) score(std::integral_constant<int, 1>{}); else score(std::integral_constant<int, 2>{});
     SPR_LAUNCHED("svg_ear_score_kernel<value>");
   } else {
-    svg_ear_score_kernel<1><<<grid, threads, 0, stream>>>(q_centroids, k_sorted, nullptr, nullptr, k_sizes, qn, kn,
-                                                          t_stored, group, qgroups, qwaves, sets, scores);
+    auto score = [&](auto step) {
+      svg_ear_score_kernel<1, decltype(step)::value><<<grid, threads, 0, stream>>>(
+          q_centroids, k_sorted, nullptr, nullptr, k_sizes, qn, kn, t_stored, group, qgroups, qwaves, sets, scores);
+    };
+    if (few) score(std::integral_constant<int, 1>{}); else score(std::integral_constant<int, 2>{});
     SPR_LAUNCHED("svg_ear_score_kernel<mass>");
   }
   return SPR_OK;

@@ -134,6 +134,33 @@ def test_value_error_scores_hold_for_large_and_small_values(dev, oracle, vscale,
     assert (np.abs(got - ref) <= ATOL + 1e-5 * np.abs(ref)).all()
 
 
+@pytest.mark.parametrize("qn", [1, 33, 64, 65, 96, 128])  # one to four query waves
+@pytest.mark.parametrize("tokens,vscale", [(1, 1.0), (1, 1e16), (7, 1.0)])  # times the clusters' sizes below
+def test_scores_of_many_heads_and_short_clusters(dev, oracle, qn, tokens, vscale):
+    """384 workgroups of clusters of less than 128 tokens on average, which share the CUs by two, and of more
+    than that, which do not from 65 rows: empty clusters, runs around one, two and three chunks, tokens past the
+    last run; three heads of 48 against the oracle.  The bound is 2e-3 and 1e-5 of the score."""
+    from sparsepr_amd.kernels.svg_ear import attention_mass_scores_triton, svg_ear_value_error_scores_triton
+
+    heads, kn = 48, 64
+    sizes = np.resize(np.array([0, 33, 1, 64, 96, 65, 32, 31, 2, 0, 7], np.int32) * tokens, (heads, kn))
+    sizes[1] = sizes[0][::-1]
+    qc, k, v, kc, vc, _ = _case(qn + tokens, heads, 1, qn, sizes)
+    k, v = _bf16_np(oracle, k), _bf16_np(oracle, (v * vscale).astype(np.float32))
+    vc = (vc * vscale).astype(np.float32)
+    dk, dv, dq, ds = to_dev(k, dev, torch.bfloat16), to_dev(v, dev, torch.bfloat16), to_dev(qc, dev), to_dev(sizes, dev)
+    got = svg_ear_value_error_scores_triton(qcentroids=dq, k_sorted=dk, v_sorted=dv, kcentroids=to_dev(kc, dev),
+                                            vcentroids=to_dev(vc, dev), kcluster_sizes=ds, gqa_group=1)
+    mass = attention_mass_scores_triton(qcentroids=dq, k_sorted=dk, kcluster_sizes=ds, gqa_group=1)
+    h = [0, 1, heads - 1]
+    for a, ref in ((got, oracle.svg_ear_value_error_scores(qc[h], k[h], v[h], kc[h], vc[h], sizes[h], 1)),
+                   (mass, oracle.attention_mass_scores(qc[h], k[h], sizes[h], 1))):
+        a = a.reshape(heads, qn, kn)[h].cpu().numpy().astype(np.float64).reshape(np.shape(ref))
+        fin = np.isfinite(ref)
+        assert (np.isneginf(a) == ~fin).all()
+        assert (np.abs(a[fin] - ref[fin]) <= ATOL + 1e-5 * np.abs(ref[fin])).all()
+
+
 def test_grouped_scores_equal_ungrouped(dev, oracle):
     from sparsepr_amd.kernels.svg_ear import (svg_ear_grouped_value_error_scores_triton,
                                               svg_ear_value_error_scores_triton)
