@@ -1003,10 +1003,13 @@ __device__ void finalize_mean(double s, int32_t count, int64_t b, int32_t cl, in
 // 118,800 rows; slices sized from the average left it to two workgroups: 204 us per update
 // against 134 us on uniform labels).
 constexpr int MEAN_SLICE = 512;
-// Up to this many points per batch one workgroup takes a whole cluster, with neither plan nor
-// finalize launch: 24 x 8,192 x 64 (128 clusters) 21 us in three launches, 15.5 in one (both with
-// 8 us of graph replay); with a seventh of the points in one cluster 24.5 and 28.
-constexpr int64_t MEAN_WHOLE_N = 8192;
+// Short inputs whose clusters average a slice or less: one workgroup takes a whole cluster, with
+// neither plan nor finalize launch (8 x 4,096 x 128, 8 to 256 clusters, call by call: 16.5 us in three,
+// 12.4 in one).  It walks a long cluster alone, so fewer clusters take the slices (4,096 points in
+// one cluster 34 us against 17, 8,192 x 64 fp32 in four 28 against 17), and so do longer inputs,
+// where a cluster that holds half the points costs more than the launches.
+constexpr int64_t MEAN_WHOLE_N = 4096;
+bool mean_takes_whole_clusters(int64_t n, int64_t k) { return n <= MEAN_WHOLE_N && n <= MEAN_SLICE * k; }
 
 // One workgroup per batch: slice_base[b][c] = the first slice of cluster c (exclusive scan of
 // ceil(rows_c / MEAN_SLICE), c = 0 .. k; capped at maxs, the slices the workspace holds, so
@@ -1604,7 +1607,7 @@ extern "C" int spr_centroid_mean(const void* x, int32_t dtype, const int32_t* so
   SPR_REQUIRE(sorted_idx && offsets && old, "spr_centroid_mean: null pointer");
   SPR_REQUIRE(n == 0 || x, "spr_centroid_mean: null x");
   SPR_REQUIRE(n < (int64_t(1) << 31), "spr_centroid_mean: n too large");
-  const bool sliced = n > MEAN_WHOLE_N;
+  const bool sliced = !mean_takes_whole_clusters(n, k);
   const int64_t maxs = mean_max_slices(n, k);
   SPR_REQUIRE(maxs < (int64_t(1) << 31), "spr_centroid_mean: too many clusters");
   const size_t need = spr_centroid_mean_workspace(batch, n, k, d);

@@ -141,6 +141,25 @@ def test_centroid_mean_of_short_inputs(dev, oracle, n, dtype, d):
     assert abs(float(res.shift.item()) - shift) <= 1e-5 * max(shift, 1.0)
 
 
+@pytest.mark.parametrize("n,k", [(512, 1), (513, 1), (4096, 8), (4096, 7), (4097, 9), (8192, 1)])
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float32, 48)])
+def test_centroid_mean_of_few_clusters(dev, oracle, n, k, dtype, d):
+    """Whole clusters up to 4,096 points and 512 per cluster, slices beyond: the float64 means bit
+    for bit on both sides, with most points in one cluster."""
+    from sparsepr_amd.flash_kmeans.kmeans_impl import centroid_update_sorted
+
+    rng = np.random.default_rng(n + k)
+    x = _gmm(oracle, rng, 2, n, d, 5)
+    labels = rng.integers(0, k, (2, n)).astype(np.int32)
+    labels[rng.random((2, n)) < 0.6] = k // 2
+    old = oracle.to_bf16(rng.standard_normal((2, k, d)).astype(np.float32))
+    res = centroid_update_sorted(to_dev(x, dev, dtype), to_dev(labels, dev), to_dev(old, dev, dtype), want_mean32=True)
+    cent, mean32, counts = oracle.centroid_update(x, labels, old, out_bf16=dtype == torch.bfloat16)
+    assert (res.mean32.cpu().numpy() == mean32).all()
+    assert (res.centroids.float().cpu().numpy() == cent).all()
+    assert (res.sizes.cpu().numpy() == counts).all()
+
+
 @pytest.mark.parametrize("iters", [1, 2, 3])  # the centroids alternate between two buffers
 @pytest.mark.parametrize("dtype,d,n", [(torch.bfloat16, 64, 500), (torch.bfloat16, 128, 9000), (torch.float32, 48, 9000)])
 def test_lloyd_in_one_call_equals_its_steps(dev, oracle, iters, dtype, d, n):
