@@ -6,7 +6,7 @@
 // start offsets that the block-sparse attention schedule and the centroid
 // update consume.  Within a cluster tokens keep ascending index order.
 //
-// Rows of up to SMALL_N labels (and up to SMALL_BINS bins): one launch, one workgroup per row.
+// Short rows of up to SMALL_BINS bins (sorts_small): one launch, one workgroup per row.
 // Longer rows, three launches:
 //   1. per (row, chunk of CHUNK tokens) label histogram in LDS;
 //   2. per row: label totals, exclusive scan over labels, per-chunk bases;
@@ -25,7 +25,8 @@ namespace {
 
 constexpr int CHUNK = 4096;
 constexpr int MAX_BINS = 8192;  // k + 1 <= MAX_BINS (32 KB of LDS counters)
-constexpr int COUNTERS = 16384;   // LDS counters of a ranking workgroup (64 KB), shared by its waves
+constexpr int COUNTERS = 16384;   // LDS counters of a ranking workgroup (64 KB), shared by its waves;
+constexpr int FEW_COUNTERS = 32768;  // 128 KB where the workgroups are at most one per CU
 constexpr int SMALL_N = 16384;    // longest row sorted by one workgroup of 16 waves ...
 constexpr int SMALL_BINS = COUNTERS / 16;  // ... whose counters fit
 
@@ -256,14 +257,18 @@ __global__ void fill_i32_kernel(int32_t* __restrict__ p, int64_t count, int32_t 
     p[i] = value;
 }
 
-// One launch instead of three; one workgroup per row is also the faster up to this length
-// (24 rows, 128 bins: 16,384 labels 20.7 us, 16,385 in three launches 22, their gaps aside).
-bool sorts_small(int64_t n, int32_t k) { return n <= SMALL_N && k + 1 <= SMALL_BINS; }
+// One launch instead of three, and with one workgroup per row the faster up to 8,192 labels (24
+// rows, 256 bins, in a graph: 8,192 labels 12.3 us, 15 in three launches; 16,384 22.3 us, 16 in three),
+// above that where the rows fill the chip (256 rows of 16,384: 43 us, 44 in three launches, with 8
+// bins 18 and 28).
+bool sorts_small(int64_t rows, int64_t n, int32_t k) {
+  return n <= (rows >= 128 ? SMALL_N : SMALL_N / 2) && k + 1 <= SMALL_BINS;
+}
 
 }  // namespace
 
 extern "C" size_t spr_argsort_labels_workspace(int64_t rows, int64_t n, int32_t k) {
-  if (sorts_small(n, k)) return 16;  // none is used
+  if (sorts_small(rows, n, k)) return 16;  // none is used
   const int64_t nchunks = spr::ceil_div(n, CHUNK);
   return static_cast<size_t>(rows * nchunks * (static_cast<int64_t>(k) + 1) * 4);
 }
@@ -292,9 +297,12 @@ extern "C" int spr_argsort_labels(const int32_t* labels, int64_t rows, int64_t n
     return SPR_EWORKSPACE;
   }
   const size_t bin_bytes = static_cast<size_t>(k + 1) * sizeof(int32_t);
-  if (sorts_small(n, k)) {
+  if (sorts_small(rows, n, k)) {
     if (n <= 4096) {
       label_sort_small_kernel<4><<<dim3(rows), 1024, 16 * bin_bytes, stream>>>(labels, static_cast<int32_t>(n), k,
+                                                                              sorted_idx, sizes, offsets);
+    } else if (n <= 8192) {
+      label_sort_small_kernel<8><<<dim3(rows), 1024, 16 * bin_bytes, stream>>>(labels, static_cast<int32_t>(n), k,
                                                                               sorted_idx, sizes, offsets);
     } else {
       label_sort_small_kernel<16><<<dim3(rows), 1024, 16 * bin_bytes, stream>>>(labels, static_cast<int32_t>(n), k,
@@ -309,15 +317,29 @@ extern "C" int spr_argsort_labels(const int32_t* labels, int64_t rows, int64_t n
   SPR_LAUNCHED("label_hist_kernel");
   label_scan_kernel<<<dim3(rows), 1024, 0, stream>>>(hist, k, nchunks, sizes, offsets);
   SPR_LAUNCHED("label_scan_kernel");
-  auto scatter = [&](auto waves) {
+  // as many waves per chunk as counters fit: a whole CU's LDS where the chunks leave CUs idle (2
+  // rows of 8,192 labels, 4,096 bins: the sort 45.8 us with two waves, 31.7 with four)
+  const int32_t counters = static_cast<int64_t>(nchunks) * rows <= 256 ? FEW_COUNTERS : COUNTERS;
+  auto scatter = [&](auto waves) -> int {
     constexpr int W = decltype(waves)::value;
-    label_scatter_kernel<W><<<dim3(nchunks, rows), W * 64, W * bin_bytes, stream>>>(labels, n, k, nchunks, hist,
-                                                                                    sorted_idx);
+    const size_t bytes = W * bin_bytes;
+    if (bytes > 65536) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&label_scatter_kernel<W>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, FEW_COUNTERS * 4);
+      if (e != hipSuccess) {
+        spr_set_error("spr_argsort_labels: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+        return SPR_ELAUNCH;
+      }
+    }
+    label_scatter_kernel<W><<<dim3(nchunks, rows), W * 64, bytes, stream>>>(labels, n, k, nchunks, hist, sorted_idx);
+    return SPR_OK;
   };
-  if (16 * (k + 1) <= COUNTERS) scatter(std::integral_constant<int, 16>{});
-  else if (8 * (k + 1) <= COUNTERS) scatter(std::integral_constant<int, 8>{});
-  else if (4 * (k + 1) <= COUNTERS) scatter(std::integral_constant<int, 4>{});
-  else scatter(std::integral_constant<int, 2>{});
+  int st;
+  if (16 * (k + 1) <= counters) st = scatter(std::integral_constant<int, 16>{});
+  else if (8 * (k + 1) <= counters) st = scatter(std::integral_constant<int, 8>{});
+  else if (4 * (k + 1) <= counters) st = scatter(std::integral_constant<int, 4>{});
+  else st = scatter(std::integral_constant<int, 2>{});
+  if (st != SPR_OK) return st;
   SPR_LAUNCHED("label_scatter_kernel");
   return SPR_OK;
 }

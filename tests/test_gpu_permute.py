@@ -178,3 +178,17 @@ def test_label_sort_with_fewer_waves(dev, k):
     idx, sizes, _ = argsort_labels(torch.from_numpy(lab).to(dev), k)
     assert (idx.cpu().numpy() == np.argsort(lab, axis=1, kind="stable")).all()
     assert (sizes.cpu().numpy() == np.stack([np.bincount(r, minlength=k) for r in lab])).all()
+
+
+@pytest.mark.parametrize("rows,n,k", [(1, 8192, 256), (1, 8193, 256), (127, 8193, 40), (128, 8193, 40),
+                                      (128, 16384, 1023), (128, 16385, 8), (85, 9001, 4096), (86, 9001, 4096),
+                                      (86, 9001, 8191), (86, 9001, 2048), (65, 16300, 1024)])
+def test_label_sort_by_rows(dev, rows, n, k):
+    """One workgroup per row up to 8,192 labels, and up to 16,384 from 128 rows; the scatter's waves
+    share 128 KB of counters up to 256 chunks, 64 KB above."""
+    from sparsepr_amd.kernels.permute import argsort_labels
+
+    lab = np.random.default_rng(rows + n + k).integers(0, k, (rows, n)).astype(np.int32)
+    idx, sizes, _ = argsort_labels(torch.from_numpy(lab).to(dev), k)
+    assert (idx.cpu().numpy() == np.argsort(lab, axis=1, kind="stable")).all()
+    assert (sizes.cpu().numpy() == np.stack([np.bincount(r, minlength=k) for r in lab])).all()
