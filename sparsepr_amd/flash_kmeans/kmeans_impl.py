@@ -186,32 +186,44 @@ def lloyd(x: torch.Tensor, n_clusters: int, max_iters: int, tol: float = 0.0,
     xs = None if x_sq is None else x_sq.to(torch.float32).contiguous()
     code = _lib.DTYPE_CODE[x.dtype]
 
-    def run(iters, init, c_sq, norms, norms_out, c_sq_out, shift):
-        """`iters` iterations from `init` in one call; returns the last centroids."""
-        out = torch.empty_like(init)
-        ws = _lib.workspace(_lib.query("spr_lloyd_workspace", B, N, K, D, code, iters), dev)
-        _lib.call("spr_lloyd", _lib.ptr(x), code, _lib.ptr(init), _lib.ptr(c_sq), _lib.ptr(norms), int(x_sq_mode),
-                  _lib.ptr(norms_out), B, N, K, D, iters, _lib.ptr(labels), _lib.ptr(sorted_idx), _lib.ptr(sizes),
-                  _lib.ptr(offsets), _lib.ptr(out), _lib.ptr(c_sq_out), _lib.ptr(mean32), _lib.ptr(shift),
-                  _lib.ptr(ws), ws.numel(), _lib.stream(dev))
-        return out
+    def run(iters, init, out, ws, ws_bytes, c_sq=None, norms=None, norms_out=None, c_sq_out=None, shift=None):
+        """`iters` iterations from `init` into `out` in one call; ws and what follows are addresses."""
+        _lib.call("spr_lloyd", _lib.ptr(x), code, _lib.ptr(init), c_sq, norms, int(x_sq_mode), norms_out, B, N, K, D,
+                  iters, _lib.ptr(labels), _lib.ptr(sorted_idx), _lib.ptr(sizes), _lib.ptr(offsets), _lib.ptr(out),
+                  c_sq_out, _lib.ptr(mean32), shift, ws, ws_bytes, _lib.stream(dev))
 
     if tol <= 0 and not verbose:
-        cent = run(max_iters, cent, None, xs, None, None, None)
-        return LloydResult(labels, cent, sizes, max_iters, sorted_idx, offsets, mean32)
-    # the stop test reads the centroid movement after every iteration: one call for each; the
-    # point norms of the first serve the later ones, as do the centroid norms of each update
-    kept = torch.empty((B, N), dtype=torch.float32, device=dev) if xs is None and max_iters > 1 else None
-    c_sq = None
+        ws_bytes = int(_lib.query("spr_lloyd_workspace", B, N, K, D, code, max_iters))
+        ws = _lib.workspace(ws_bytes, dev)
+        out = torch.empty_like(cent)
+        run(max_iters, cent, out, _lib.ptr(ws), ws_bytes, norms=_lib.ptr(xs))
+        return LloydResult(labels, out, sizes, max_iters, sorted_idx, offsets, mean32)
+    # The stop test reads the centroid movement after every iteration: one call for each; the point
+    # norms of the first serve the later ones, as do the centroid norms of each update.  The GPU
+    # waits for the host between two of them, so nothing is allocated there: one buffer holds the
+    # calls' workspace, the point norms and two sets of centroid norms, and the centroids alternate.
+    def aligned(nbytes):
+        return (int(nbytes) + 255) // 256 * 256
+
+    ws_bytes = aligned(_lib.query("spr_lloyd_workspace", B, N, K, D, code, 1))
+    kept_bytes = aligned(4 * B * N) if xs is None and max_iters > 1 else 0
+    scratch = _lib.workspace(ws_bytes + kept_bytes + 2 * aligned(4 * B * K), dev)
+    ws = _lib.ptr(scratch)
+    kept = ws + ws_bytes if kept_bytes else None
+    c_sqs = [ws + ws_bytes + kept_bytes + i * aligned(4 * B * K) for i in (0, 1)]
+    shifts = torch.zeros(max_iters, dtype=torch.float32, device=dev)
+    outs = [torch.empty_like(cent)]
     for it in range(max_iters):
-        norms = xs if xs is not None else (kept if it > 0 else None)
-        c_sq_out = torch.empty((B, K), dtype=torch.float32, device=dev)
-        shift = torch.zeros(1, dtype=torch.float32, device=dev)
-        new = run(1, cent, c_sq, norms, kept if norms is None else None, c_sq_out, shift)
-        moved = float(shift.item())
+        norms = _lib.ptr(xs) if xs is not None else (kept if it > 0 else None)
+        new = outs[it % 2]
+        run(1, cent, new, ws, ws_bytes, c_sqs[(it + 1) % 2] if it > 0 else None, norms, kept if norms is None else None,
+            c_sqs[it % 2], _lib.ptr(shifts) + 4 * it)
+        if it == 0 and max_iters > 1:
+            outs.append(torch.empty_like(cent))
+        moved = float(shifts[it].item())
         if verbose:
             print(f"Iter {it}, center shift: {moved:.6f}")
         if tol > 0 and moved < tol:
             return LloydResult(labels, cent, sizes, it + 1, sorted_idx, offsets, mean32)
-        cent, c_sq = new, c_sq_out
+        cent = new
     return LloydResult(labels, cent, sizes, max_iters, sorted_idx, offsets, mean32)
