@@ -111,8 +111,8 @@ int spr_centroid_mean(const void* x, int32_t dtype, const int32_t* sorted_idx, c
  * (nullable: computed) are init's squared norms; x_sq, x_sq_mode and x_sq_out as for
  * spr_kmeans_assign_bf16 (without x_sq the first iteration's norms serve the later ones).
  * Outputs: labels, sorted_idx, sizes and offsets of the last assignment, cent [batch,k,d] (not
- * init's buffer) of the last update, and, nullable, its c_sq_out, mean32 and shift_max as
- * spr_centroid_mean writes them. */
+ * init's buffer) of the last update, and, nullable, its c_sq_out, mean32 and shift_max (which need
+ * not be zero) as spr_centroid_mean writes them. */
 size_t spr_lloyd_workspace(int64_t batch, int64_t n, int32_t k, int32_t d, int32_t dtype, int32_t iters);
 int spr_lloyd(const void* x, int32_t dtype, const void* init, const float* c_sq, const float* x_sq, int32_t x_sq_mode,
               float* x_sq_out, int64_t batch, int64_t n, int32_t k, int32_t d, int32_t iters, int32_t* labels,

@@ -1690,6 +1690,9 @@ LloydSpace lloyd_space(int64_t batch, int64_t n, int32_t k, int32_t d, int32_t d
   w.x_sq = take(iters > 1 ? static_cast<size_t>(batch) * n * sizeof(float) : 0);
   return w;
 }
+__global__ void zero_f32_kernel(float* __restrict__ p) {
+  if (threadIdx.x == 0) *p = 0.0f;
+}
 }  // namespace
 
 extern "C" size_t spr_lloyd_workspace(int64_t batch, int64_t n, int32_t k, int32_t d, int32_t dtype, int32_t iters) {
@@ -1735,9 +1738,13 @@ extern "C" int spr_lloyd(const void* x, int32_t dtype, const void* init, const f
                     : spr_kmeans_assign_tf32(static_cast<const float*>(x), static_cast<const float*>(old), c_sq, xs, xo,
                                              batch, n, k, d, labels, stream);
     if (st != SPR_OK) return st;
+    const bool last = it + 1 == iters;
+    if (last && shift_max != nullptr) {  // behind the assignment, which keeps the GPU busy meanwhile
+      zero_f32_kernel<<<1, 64, 0, stream>>>(shift_max);
+      SPR_LAUNCHED("zero_f32_kernel");
+    }
     st = spr_argsort_labels(labels, batch, n, k, sorted_idx, sizes, offsets, ws + w.sort, w.sort_bytes, stream);
     if (st != SPR_OK) return st;
-    const bool last = it + 1 == iters;
     void* next = buffers[(iters - 1 - it) % 2];
     float* next_sq = last && c_sq_out != nullptr ? c_sq_out : norms[it % 2];
     st = spr_centroid_mean(x, dtype, sorted_idx, offsets, old, batch, n, k, d, last ? mean32 : nullptr, next,

@@ -211,16 +211,16 @@ def lloyd(x: torch.Tensor, n_clusters: int, max_iters: int, tol: float = 0.0,
     ws = _lib.ptr(scratch)
     kept = ws + ws_bytes if kept_bytes else None
     c_sqs = [ws + ws_bytes + kept_bytes + i * aligned(4 * B * K) for i in (0, 1)]
-    shifts = torch.zeros(max_iters, dtype=torch.float32, device=dev)
+    shift = torch.empty(1, dtype=torch.float32, device=dev)
     outs = [torch.empty_like(cent)]
     for it in range(max_iters):
         norms = _lib.ptr(xs) if xs is not None else (kept if it > 0 else None)
         new = outs[it % 2]
         run(1, cent, new, ws, ws_bytes, c_sqs[(it + 1) % 2] if it > 0 else None, norms, kept if norms is None else None,
-            c_sqs[it % 2], _lib.ptr(shifts) + 4 * it)
+            c_sqs[it % 2], _lib.ptr(shift))
         if it == 0 and max_iters > 1:
             outs.append(torch.empty_like(cent))
-        moved = float(shifts[it].item())
+        moved = float(shift.item())
         if verbose:
             print(f"Iter {it}, center shift: {moved:.6f}")
         if tol > 0 and moved < tol:
