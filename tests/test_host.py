@@ -133,12 +133,13 @@ def test_tile_order_deals_every_tile_once_and_the_longest_early(tmp_path):
     """Every tile of every head has one workgroup, with few to spare, and list scheduling on 8 XCDs
     of 32 workgroups ends near the ideal: with a prompt, whose query tiles keep every key and so walk
     1 / density = 5 times the chunks, and without one."""
-    edges = [(rows, most, heads) for rows, most in ((1, 2), (7, 9), (16, 17), (79, 130), (80, 81), (465, 765))
+    edges = [(rows, most, heads) for rows, most in ((1, 2), (7, 9), (16, 17), (31, 33), (32, 33), (79, 130), (127, 128), (128, 161),
+                                                       (465, 765))
              for heads in (1, 2, 7, 8, 9, 24, 300)]
     for (rows, most, heads), order in zip(edges, _tile_orders(tmp_path, edges)):
         got = order[(order[:, 0] < heads) & (order[:, 1] < most)]
         assert len(got) == heads * most and len(np.unique(got, axis=0)) == heads * most
-        run = 8 if rows >= 256 else 4 if rows >= 32 else 2
+        run = 8 if rows >= 128 else 4 if rows >= 32 else 2
         assert len(order) <= heads * (most + 4 * run) + 16 * run  # two parts, each an odd number of runs
     rng = np.random.default_rng(0)
     cases = [(heads, tokens, text) for heads in (3, 5, 8, 12, 16, 24) for tokens in (20000, 35400, 60000, 118800)
