@@ -1355,16 +1355,18 @@ constexpr int TO_MAX_QN = 4096;  // q-clusters per head the tile order handles i
 // One more workgroup orders the heads by decreasing work, sum over q-clusters of 256-row tiles x
 // 64-key chunks (ties by index): the heads follow one another over the tile grid, and a call
 // should end on a light one (16 heads of 35,400 tokens whose densities differ by up to 4: 2.81 ms
-// in index order, 2.69 so).  Identity where the terms are many: above HO_MAX heads or
-// HO_TERMS (head, q-cluster) pairs it would take longer than the others, and a call of so many
-// heads ends evenly.
+// in index order, 2.69 so).  Identity from HO_ROWS rows on, where a head fills the chip by itself
+// and the order costs (24 x 118,800: 32.1 ms in index order, 32.5 so), and where the terms are many:
+// above HO_MAX heads or HO_TERMS (head, q-cluster) pairs it would take longer than the others, and a
+// call of so many heads ends evenly.
+constexpr int HO_ROWS = 65536;
 constexpr int HO_MAX = 1024;
 constexpr int HO_TERMS = 32768;
-__device__ void write_head_order(int32_t* plan, int32_t bh_kv, int32_t qn, int32_t kn) {
+__device__ void write_head_order(int32_t* plan, int32_t bh_kv, int32_t qn, int32_t kn, int32_t s) {
   __shared__ unsigned long long work[HO_MAX];
   int32_t* order = head_order_at(plan, bh_kv, qn, kn);
   const int tid = threadIdx.x;
-  if (bh_kv > HO_MAX || static_cast<int64_t>(bh_kv) * qn > HO_TERMS) {
+  if (s >= HO_ROWS || bh_kv > HO_MAX || static_cast<int64_t>(bh_kv) * qn > HO_TERMS) {
     for (int h = tid; h < bh_kv; h += blockDim.x) order[h] = h;
     return;
   }
@@ -1389,7 +1391,7 @@ __global__ __launch_bounds__(256) void attn_tile_order_kernel(int32_t* __restric
   extern __shared__ int32_t to_lds[];  // total[qn], tiles[qn], by_len[qn]
   const int32_t bh_kv = static_cast<int32_t>(gridDim.x) - 1;
   if (static_cast<int32_t>(blockIdx.x) == bh_kv) {
-    write_head_order(plan, bh_kv, qn, kn);
+    write_head_order(plan, bh_kv, qn, kn, s);
     return;
   }
   int32_t* tl = to_lds;
