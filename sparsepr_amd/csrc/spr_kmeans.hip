@@ -1003,13 +1003,16 @@ __device__ void finalize_mean(double s, int32_t count, int64_t b, int32_t cl, in
 // 118,800 rows; slices sized from the average left it to two workgroups: 204 us per update
 // against 134 us on uniform labels).
 constexpr int MEAN_SLICE = 512;
-// Short inputs whose clusters average a slice or less: one workgroup takes a whole cluster, with
-// neither plan nor finalize launch (8 x 4,096 x 128, 8 to 256 clusters, call by call: 16.5 us in three,
-// 12.4 in one).  It walks a long cluster alone, so fewer clusters take the slices (4,096 points in
-// one cluster 34 us against 17, 8,192 x 64 fp32 in four 28 against 17), and so do longer inputs,
-// where a cluster that holds half the points costs more than the launches.
+// Short inputs with many clusters: one workgroup takes a whole cluster, with neither plan nor
+// finalize launch.  It walks a long cluster alone, so the clusters have to be short even where a
+// few hold several times the average: at most 128 rows on average, fp32 rows (half as many to a
+// pass) 64, or 1,024 in all.  In a graph, 15 x 4,096 points, sizes of a log-normal of 0.8, in three
+// launches and in one: 128 dims bf16, 82 clusters 13.7 us and 8.3, 21 clusters 13 and up to 25, 9
+// clusters 14 and 39; 64 dims fp32, 32 clusters 13.5 and 15.5.
 constexpr int64_t MEAN_WHOLE_N = 4096;
-bool mean_takes_whole_clusters(int64_t n, int64_t k) { return n <= MEAN_WHOLE_N && n <= MEAN_SLICE * k; }
+bool mean_takes_whole_clusters(int64_t n, int64_t k, int32_t dtype) {
+  return n <= 1024 || (n <= MEAN_WHOLE_N && n <= (dtype == 0 ? 128 : 64) * k);
+}
 
 // One workgroup per batch: slice_base[b][c] = the first slice of cluster c (exclusive scan of
 // ceil(rows_c / MEAN_SLICE), c = 0 .. k; capped at maxs, the slices the workspace holds, so
@@ -1607,7 +1610,7 @@ extern "C" int spr_centroid_mean(const void* x, int32_t dtype, const int32_t* so
   SPR_REQUIRE(sorted_idx && offsets && old, "spr_centroid_mean: null pointer");
   SPR_REQUIRE(n == 0 || x, "spr_centroid_mean: null x");
   SPR_REQUIRE(n < (int64_t(1) << 31), "spr_centroid_mean: n too large");
-  const bool sliced = !mean_takes_whole_clusters(n, k);
+  const bool sliced = !mean_takes_whole_clusters(n, k, dtype);
   const int64_t maxs = mean_max_slices(n, k);
   SPR_REQUIRE(maxs < (int64_t(1) << 31), "spr_centroid_mean: too many clusters");
   const size_t need = spr_centroid_mean_workspace(batch, n, k, d);

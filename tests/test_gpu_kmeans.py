@@ -141,11 +141,12 @@ def test_centroid_mean_of_short_inputs(dev, oracle, n, dtype, d):
     assert abs(float(res.shift.item()) - shift) <= 1e-5 * max(shift, 1.0)
 
 
-@pytest.mark.parametrize("n,k", [(512, 1), (513, 1), (4096, 8), (4096, 7), (4097, 9), (8192, 1)])
+@pytest.mark.parametrize("n,k", [(1024, 1), (1025, 1), (4096, 64), (4096, 63), (4096, 32), (4096, 31), (4097, 70),
+                                 (8192, 1)])
 @pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float32, 48)])
 def test_centroid_mean_of_few_clusters(dev, oracle, n, k, dtype, d):
-    """Whole clusters up to 4,096 points and 512 per cluster, slices beyond: the float64 means bit
-    for bit on both sides, with most points in one cluster."""
+    """Whole clusters up to 1,024 points, up to 4,096 at 128 (fp32 64) per cluster, slices beyond:
+    the float64 means bit for bit on both sides, with most points in one cluster."""
     from sparsepr_amd.flash_kmeans.kmeans_impl import centroid_update_sorted
 
     rng = np.random.default_rng(n + k)
