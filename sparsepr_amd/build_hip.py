@@ -26,7 +26,7 @@ FLAGS = [
     "-fPIC",
     "-Wall",
     "-Wno-unused-function",
-    # packed FP32 instructions are disabled for all device code on this pool
+    # packed FP32 instructions are disabled for all device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 

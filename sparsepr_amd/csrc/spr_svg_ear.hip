@@ -17,8 +17,7 @@
 //   attention mass: score = log(max(sum_t e^(l_t - m), 1e-30)) + m, m = max_t l_t
 // The weights are taken against a reference that starts at l_c (the mass: at the first
 // chunk's maximum) and moves only when a logit passes it by SE_SLACK (less where |v|^2 is large),
-// with the sums rescaled;
-// the scores do not depend on it but for rounding.
+// with the sums rescaled; the scores do not depend on it but for rounding.
 //
 // Layout.  A first kernel writes the centroid logits l_c [query head, centroid, cluster]
 // (fp32 dot products over d, sequential, 128 rows x 32 clusters per workgroup) into the score
@@ -27,23 +26,23 @@
 // per 32-row query block (two for up to five blocks, each folding every other chunk), two
 // waves for the statistics of V, at most twelve, three per SIMD.  K and V are walked once for
 // all rows.  Calls of up to 128 rows with many short clusters take four waves, one chunk per
-// barrier and half the LDS, two workgroups per CU (the host's rule).  The clusters' tokens are one contiguous run, walked in 32-token chunks (a chunk
-// never spans two clusters), whose K and V rows are DMA'd into swizzled LDS tiles (16-byte
-// piece p of token row t at slot p ^ (t % 16): the MFMA fragment reads hit 16 distinct slots
-// per 16 lanes) two steps ahead.  A query wave forms S^T = K Q~^T by 16 bf16
-// MFMAs per chunk: q~ is split into bf16 hi + lo with hi + lo == q~ exactly (q~ has 11
+// barrier and half the LDS, two workgroups per CU (the host's rule).  The clusters' tokens are one
+// contiguous run, walked in 32-token chunks (a chunk never spans two clusters), whose K and V rows
+// are DMA'd into swizzled LDS tiles (16-byte piece p of token row t at slot p ^ (t % 16): the MFMA
+// fragment reads hit 16 distinct slots per 16 lanes) two steps ahead.  A query wave forms
+// S^T = K Q~^T by 16 bf16 MFMAs per chunk: q~ is split into bf16 hi + lo with hi + lo == q~ exactly (q~ has 11
 // significant bits, hi the top 8, lo the next 3), so every product is the reference's TF32
 // product exactly and only the fp32 summation order differs.  |v_t|^2 and v_t . vc are products
 // of the V tile with itself and with the three bf16 pieces of vc, a chunk ahead of their use.
 //
 // What bounds it: the folding, 5 VALU operations, an exponential (16 cycles) and half a max
 // per (centroid, token) pair beside the MFMAs, which a wave does not overlap with its own
-// (computing S a chunk ahead needs more registers than three waves per SIMD have).  24 heads x
-// 118,800 tokens, 300 x 1000: 1.27 -> 0.94 ms; 180 x 512 at 70,000 tokens (both kernels) 0.64
-// -> 0.48 ms, 128 x 512 at 118,800 0.55 -> 0.53 ms, 6 heads x 9,000 tokens, 23 x 64: 105 -> 64
-// us, against four waves per 128 rows that walked K and V again for every 128 rows and took
-// the statistics of V on all their lanes.  One wave for the statistics instead of two holds
-// the others up (128 x 512: 0.64 ms); one chunk per barrier costs 5 %.
+// (computing S a chunk ahead needs more registers than three waves per SIMD have, and with two to
+// a CU it changed nothing).  Both kernels, against four waves per 128 rows that walked K and V again
+// for every 128 rows and took the statistics of V on all their lanes: 24 heads x 118,800 tokens,
+// 300 x 1000 1.37 -> 1.02 ms; 180 x 512 at 70,000 tokens 0.61 -> 0.46 ms; 128 x 512 at 118,800 0.51
+// -> 0.51 ms; 6 heads x 9,000 tokens, 23 x 64 99 -> 61 us.  One wave for the statistics instead of
+// two holds the others up (128 x 512: 0.64 ms); one chunk per barrier costs 5 %.
 // The token runs come from a block prefix sum of the sizes and are clamped to the stored
 // tokens, so no size vector can make the kernel read outside K or V.
 #include <type_traits>
@@ -856,7 +855,7 @@ extern "C" int spr_svg_ear_scores(const float* q_centroids, const uint16_t* k_so
   // that two share it, where there are 1.5 or more for each CU and the clusters are short enough
   // (in long ones the second chunk per barrier and the two sets of query waves are worth more).
   // 24 heads x 40,000 tokens, 64 rows: 1,000 clusters 284 -> 216 us, 134 clusters 184 -> 180;
-  // 118,800 tokens, 134 clusters 440 -> 461.  128 rows: 1,000 clusters 331 -> 276 us, 300
+  // 118,800 tokens, 134 clusters (not short) 440 -> 461.  128 rows: 1,000 clusters 331 -> 276 us, 300
   // clusters 226 -> 230.  8 heads x 40,000 tokens (304 workgroups), 64 rows: 92 -> 98 us.
   const int32_t qblocks = (qn + 31) / 32;
   const int64_t cluster_tokens = mode == 0 && qblocks > 2 ? 128 : 512;  // mean of the longest that are short
