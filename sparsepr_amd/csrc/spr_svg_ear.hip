@@ -854,13 +854,19 @@ extern "C" int spr_svg_ear_scores(const float* q_centroids, const uint16_t* k_so
   // tiles.  Up to four blocks leave most of a CU idle: its workgroups then take half the LDS, so
   // that two share it, where there are 1.5 or more for each CU and the clusters are short enough
   // (in long ones the second chunk per barrier and the two sets of query waves are worth more).
-  // 24 heads x 40,000 tokens, 64 rows: 1,000 clusters 284 -> 216 us, 134 clusters 184 -> 180;
-  // 118,800 tokens, 134 clusters (not short) 440 -> 461.  128 rows: 1,000 clusters 331 -> 276 us, 300
-  // clusters 226 -> 230.  8 heads x 40,000 tokens (304 workgroups), 64 rows: 92 -> 98 us.
+  // Up to two blocks, 24 heads x 40,000 tokens, 64 rows: 1,000 clusters 284 -> 216 us, 134 clusters
+  // 184 -> 180; 118,800 tokens, 134 clusters (not short) 440 -> 461; 8 heads x 40,000 tokens (304
+  // workgroups), 64 rows: 92 -> 98 us.  Three and four blocks of value error leave the statistics no
+  // wave of their own, so only short clusters gain, and longer ones where three or more workgroups
+  // per CU fill the turns.  Speed against whole workgroups, 97 to 128 rows: clusters of 24 tokens
+  // 1.03 to 1.23, of 40 0.98 to 1.11 (from 768 workgroups on 1.12 to 1.18), of 90 0.94 to 0.97 (0.99
+  // to 1.08), of 221 at 475 workgroups 0.82; 65 to 96 rows: of 24 0.98 to 1.13, of 40 0.91 to 0.94
+  // (1.05), of 90 0.83 to 0.88 (0.93 to 1.02).
   const int32_t qblocks = (qn + 31) / 32;
-  const int64_t cluster_tokens = mode == 0 && qblocks > 2 ? 128 : 512;  // mean of the longest that are short
-  const bool few = qblocks <= Step<1>::QWAVES && spr::ceil_div(kn, SE_CPW) * q_heads >= 384 &&
-                   t_stored <= cluster_tokens * kn;
+  const int64_t groups = spr::ceil_div(kn, SE_CPW) * q_heads;
+  const int64_t cluster_tokens =  // mean of the longest that are short
+      mode != 0 || qblocks <= 2 ? 512 : (qblocks == 3 ? 24 : 48) * (groups >= 768 ? 2 : 1);
+  const bool few = qblocks <= Step<1>::QWAVES && groups >= 384 && t_stored <= cluster_tokens * kn;
   const int32_t most = few ? Step<1>::QWAVES : Step<2>::QWAVES;
   const int32_t qgroups = (qblocks + most - 1) / most;
   const int32_t qwaves = (qblocks + qgroups - 1) / qgroups;

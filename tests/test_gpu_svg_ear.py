@@ -135,14 +135,15 @@ def test_value_error_scores_hold_for_large_and_small_values(dev, oracle, vscale,
 
 
 @pytest.mark.parametrize("qn", [1, 33, 64, 65, 96, 128])  # one to four query waves
-@pytest.mark.parametrize("tokens,vscale", [(1, 1.0), (1, 1e16), (7, 1.0)])  # times the clusters' sizes below
-def test_scores_of_many_heads_and_short_clusters(dev, oracle, qn, tokens, vscale):
-    """384 workgroups of clusters of less than 128 tokens on average, which share the CUs by two, and of more
-    than that, which do not from 65 rows: empty clusters, runs around one, two and three chunks, tokens past the
-    last run; three heads of 48 against the oracle.  The bound is 2e-3 and 1e-5 of the score."""
+@pytest.mark.parametrize("heads,tokens,vscale", [(48, 1, 1.0), (48, 1, 1e16), (48, 7, 1.0),  # times the clusters'
+                                                 (96, 1, 1.0), (96, 1, 1e16)])  # sizes below
+def test_scores_of_many_heads_and_short_clusters(dev, oracle, qn, heads, tokens, vscale):
+    """384 and 768 workgroups of clusters of 30 tokens on average, which share the CUs by two (of the 384 those of
+    three query waves do not), and of 210, which do not from 65 rows: empty clusters, runs around one, two and three
+    chunks, tokens past the last run; three of the heads against the oracle.  The bound is 2e-3 and 1e-5 of the score."""
     from sparsepr_amd.kernels.svg_ear import attention_mass_scores_triton, svg_ear_value_error_scores_triton
 
-    heads, kn = 48, 64
+    kn = 64
     sizes = np.resize(np.array([0, 33, 1, 64, 96, 65, 32, 31, 2, 0, 7], np.int32) * tokens, (heads, kn))
     sizes[1] = sizes[0][::-1]
     qc, k, v, kc, vc, _ = _case(qn + tokens, heads, 1, qn, sizes)
